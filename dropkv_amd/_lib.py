@@ -55,6 +55,11 @@ _SIGNATURES = {
                                  _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
                                  _c_float, _c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_i64,
                                  _c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_vp, _c_size, _c_vp]),
+    "dropkv_evict_strided": (_c_int, [_c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_i64,
+                                      _c_vp, _c_i64, _c_i64, _c_i64, _c_int,
+                                      _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+                                      _c_float, _c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_i64,
+                                      _c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_vp, _c_size, _c_vp]),
     "dropkv_append": (_c_int, [_c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
                                _c_vp, _c_vp, _c_i64, _c_i64, _c_vp]),
     "dropkv_set_tail_select": (_c_int, [_c_int, _c_i64, _c_i64]),

@@ -40,6 +40,11 @@ bool decode_head_dim_supported(int64_t D) { return D == 64 || D == 128; }
 
 int64_t elem_size(int dtype) { return dtype == DROPKV_FP32 ? 4 : 2; }
 
+// K/V of [B, Hkv, ld, D] buffers.
+dkv::KvSrc dense_kv(const void* k, const void* v, int64_t ld, int64_t Hkv, int64_t D) {
+  return dkv::KvSrc{k, v, Hkv * ld * D, ld * D, D, Hkv * ld * D, ld * D, D};
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Whether the plan's 32-bit counts hold: query rows B*Hq*W (the generic
@@ -131,8 +136,8 @@ int dropkv_scores(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64
   if (!workspace || workspace_bytes < p.total)
     return fail(DROPKV_E_WORKSPACE, "workspace too small: need %zu bytes, got %zu", p.total, workspace_bytes);
   timing_start(static_cast<hipStream_t>(stream));
-  return hip_status(dkv::launch_scores(p, dtype, (int)D, q, q_sb, q_sh, q_ss, q_sd, k, v, (int)Lk,
-                                       (int)Hkv, (int)Lq, (int)Lk, (int)W, eps, p_round ? 1 : 0, y_round ? 1 : 0, scores,
+  return hip_status(dkv::launch_scores(p, dtype, (int)D, q, q_sb, q_sh, q_ss, q_sd,
+                                       dense_kv(k, v, Lk, Hkv, D), (int)Hkv, (int)Lq, (int)Lk, (int)W, eps, p_round ? 1 : 0, y_round ? 1 : 0, scores,
                                        static_cast<char*>(workspace), nullptr, 0, nullptr,
                                        static_cast<hipStream_t>(stream)),
                     "dropkv_scores launch");
@@ -231,21 +236,20 @@ size_t dropkv_evict_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t 
 }
 
 
-// One layer-call on K/V of [B*Hkv, kv_ld, D] (rows 0 .. Lk-1 used) into
+// One layer-call on K/V by strides (rows 0 .. Lk-1 of each head) into
 // outputs of [B*Hkv, out_ld, D] (rows 0 .. keep-1 written).
-static int evict_impl(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd, const void* k, const void* v,
-               int64_t kv_ld, int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Lq, int64_t Lk, int64_t D,
+static int evict_impl(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd, const dkv::KvSrc& kv,
+               int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Lq, int64_t Lk, int64_t D,
                int64_t W, float eps, int p_round, int y_round, int64_t splits, int64_t kernel_size,
                int64_t protect_window, int64_t keep, float* scores, int64_t* keep_idx, void* k_out, void* v_out,
                int64_t out_ld, void* workspace, size_t workspace_bytes, void* stream) {
   (void)hipGetLastError();  // a failure left by an unrelated earlier call is not ours
-  int rc = check_score_args(q, k, v, dtype, B, Hq, Hkv, Lq, Lk, D, W);
+  int rc = check_score_args(q, kv.k, kv.v, dtype, B, Hq, Hkv, Lq, Lk, D, W);
   if (rc) return rc;
   rc = check_select_args(reinterpret_cast<const float*>(1), B * Hkv, Lk, kernel_size, protect_window, keep, keep_idx);
   if (rc) return rc;
   if (!k_out || !v_out) return fail(DROPKV_E_ARG, "null k_out/v_out pointer");
-  if (kv_ld < Lk || out_ld < keep) return fail(DROPKV_E_ARG, "row capacity below the rows used");
-  if (kv_ld > INT32_MAX) return fail(DROPKV_E_UNSUPPORTED, "row capacity too large");
+  if (out_ld < keep) return fail(DROPKV_E_ARG, "row capacity below the rows used");
   const dkv::ScorePlan p = dkv::make_score_plan(B, Hq, Hkv, Lk, D, W, splits);
   const size_t s_bytes = ((size_t)B * Hkv * Lk * 4 + 255) & ~size_t(255);
   const size_t need = p.total + s_bytes + dkv::select_workspace_bytes(B * Hkv, Lk);
@@ -262,7 +266,7 @@ static int evict_impl(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, i
   if (!vec && out_ld != keep)
     return fail(DROPKV_E_UNSUPPORTED, "outputs with a row capacity need 16-byte aligned rows");
   timing_start(st);
-  const dkv::SelectCompact cp{k, v, Hkv * kv_ld * D, kv_ld * D, D, eb, D, (int)Hkv, k_out, v_out, out_ld};
+  const dkv::SelectCompact cp{kv, eb, D, (int)Hkv, k_out, v_out, out_ld};
   // Pooling runs in the tail of the scoring pass when the plan allows it
   // (the matrix-core kernels only); otherwise as the standalone selection's
   // pool kernel.  Where pass 2 cannot run the whole selection in its tail,
@@ -272,8 +276,8 @@ static int evict_impl(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, i
   int tail_done = 0;
   const dkv::FuseSelect fs{sel_ws,   (int)kernel_size,        (int)protect_window, (int)keep,
                            keep_idx, vec ? &cp : nullptr, &tail_done};
-  hipError_t e = dkv::launch_scores(p, dtype, (int)D, q, q_sb, q_sh, q_ss, q_sd, k, v, (int)kv_ld, (int)Hkv, (int)Lq,
-                                    (int)Lk, (int)W, eps, p_round ? 1 : 0, y_round ? 1 : 0, sc, ws,
+  hipError_t e = dkv::launch_scores(p, dtype, (int)D, q, q_sb, q_sh, q_ss, q_sd, kv, (int)Hkv, (int)Lq, (int)Lk,
+                                    (int)W, eps, p_round ? 1 : 0, y_round ? 1 : 0, sc, ws,
                                     reinterpret_cast<uint32_t*>(sel_ws), dkv::select_zero_words(B * Hkv),
                                     fused ? &fs : nullptr, st);
   if (e != hipSuccess) return hip_status(e, "dropkv_evict scores");
@@ -287,7 +291,8 @@ static int evict_impl(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, i
                            nullptr, sel_ws, true, vec ? &cp : nullptr, st);
   if (e != hipSuccess) return hip_status(e, "dropkv_evict select");
   if (vec) return DROPKV_OK;
-  e = dkv::launch_compact(k, v, Hkv * kv_ld * D, kv_ld * D, D, Lk, nullptr, nullptr, 0, 0, 0, 0, eb, B, Hkv, D,
+  // (Rows that do not allow 16-byte copies come dense: K and V alike.)
+  e = dkv::launch_compact(kv.k, kv.v, kv.k_sb, kv.k_sh, kv.k_sl, Lk, nullptr, nullptr, 0, 0, 0, 0, eb, B, Hkv, D,
                           keep_idx, keep, k_out, v_out, st);
   return hip_status(e, "dropkv_evict compact");
 }
@@ -297,7 +302,7 @@ int dropkv_evict(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_
                  float eps, int p_round, int y_round, int64_t splits, int64_t kernel_size, int64_t protect_window,
                  int64_t keep, float* scores, int64_t* keep_idx, void* k_out, void* v_out, void* workspace,
                  size_t workspace_bytes, void* stream) {
-  return evict_impl(q, q_sb, q_sh, q_ss, q_sd, k, v, Lk, dtype, B, Hq, Hkv, Lq, Lk, D, W, eps, p_round, y_round,
+  return evict_impl(q, q_sb, q_sh, q_ss, q_sd, dense_kv(k, v, Lk, Hkv, D), dtype, B, Hq, Hkv, Lq, Lk, D, W, eps, p_round, y_round,
                     splits, kernel_size, protect_window, keep, scores, keep_idx, k_out, v_out, keep, workspace,
                     workspace_bytes, stream);
 }
@@ -361,7 +366,7 @@ int dropkv_evict_noalloc(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss
   void* ws = nullptr;
   rc = noalloc_scratch(static_cast<hipStream_t>(stream), &ws);
   if (rc) return rc;
-  return evict_impl(q, q_sb, q_sh, q_ss, q_sd, k, v, Lk, dtype, B, Hq, Hkv, Lq, Lk, D, W, eps, p_round, y_round,
+  return evict_impl(q, q_sb, q_sh, q_ss, q_sd, dense_kv(k, v, Lk, Hkv, D), dtype, B, Hq, Hkv, Lq, Lk, D, W, eps, p_round, y_round,
                     splits, kernel_size, protect_window, keep, scores, keep_idx, k_out, v_out, keep, ws,
                     DROPKV_NOALLOC_SCRATCH_BYTES, stream);
 }
@@ -372,9 +377,38 @@ int dropkv_evict_ld(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int
                     int64_t kernel_size, int64_t protect_window, int64_t keep, float* scores, int64_t* keep_idx,
                     void* k_out, void* v_out, int64_t out_ld, void* workspace, size_t workspace_bytes,
                     void* stream) {
-  return evict_impl(q, q_sb, q_sh, q_ss, q_sd, k, v, kv_ld, dtype, B, Hq, Hkv, Lq, Lk, D, W, eps, p_round, y_round,
+  if (kv_ld < Lk || out_ld < keep) return fail(DROPKV_E_ARG, "row capacity below the rows used");
+  if (kv_ld > INT32_MAX) return fail(DROPKV_E_UNSUPPORTED, "row capacity too large");
+  return evict_impl(q, q_sb, q_sh, q_ss, q_sd, dense_kv(k, v, kv_ld, Hkv, D), dtype, B, Hq, Hkv, Lq, Lk, D, W, eps, p_round, y_round,
                     splits, kernel_size, protect_window, keep, scores, keep_idx, k_out, v_out, out_ld, workspace,
                     workspace_bytes, stream);
+}
+
+int dropkv_evict_strided(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd, const void* k,
+                         int64_t k_sb, int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh,
+                         int64_t v_sl, int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Lq, int64_t Lk,
+                         int64_t D, int64_t W, float eps, int p_round, int y_round, int64_t splits,
+                         int64_t kernel_size, int64_t protect_window, int64_t keep, float* scores,
+                         int64_t* keep_idx, void* k_out, void* v_out, int64_t out_ld, void* workspace,
+                         size_t workspace_bytes, void* stream) {
+  // Rows of another spacing than D: whole 16-byte units apart (the vector
+  // loads) and within the kernels' 32-bit row offsets.
+  if (dtype == DROPKV_BF16 || dtype == DROPKV_FP16 || dtype == DROPKV_FP32) {
+    const int64_t eb = elem_size(dtype);
+    const bool dense = k_sl == D && v_sl == D && k_sh == Lk * D && v_sh == Lk * D && k_sb == Hkv * Lk * D &&
+                       v_sb == Hkv * Lk * D;
+    const int64_t strides[] = {k_sb, k_sh, k_sl, v_sb, v_sh, v_sl};
+    for (const int64_t s : strides)
+      if (!dense && (s < 0 || (s * eb) % 16 != 0))
+        return fail(DROPKV_E_UNSUPPORTED, "K/V strides must be whole 16-byte units, or K and V dense");
+    if (!dense && ((D * eb) % 16 != 0 || !aligned16(k_out) || !aligned16(v_out)))
+      return fail(DROPKV_E_UNSUPPORTED, "K/V that are not dense need rows and outputs of whole 16-byte units");
+    if (!dense && (!dkv::kv_rows_fit(k_sl, eb, Lk, D) || !dkv::kv_rows_fit(v_sl, eb, Lk, D)))
+      return fail(DROPKV_E_UNSUPPORTED, "K/V rows overlap or lie too far apart");
+  }
+  return evict_impl(q, q_sb, q_sh, q_ss, q_sd, dkv::KvSrc{k, v, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl}, dtype, B, Hq,
+                    Hkv, Lq, Lk, D, W, eps, p_round, y_round, splits, kernel_size, protect_window, keep, scores,
+                    keep_idx, k_out, v_out, out_ld, workspace, workspace_bytes, stream);
 }
 
 int dropkv_append(const void* k, const void* v, int64_t s_b, int64_t s_h, int64_t s_l, int64_t elem_bytes,

@@ -49,7 +49,7 @@ __device__ __forceinline__ float gen_logit(const float* qs, const T* __restrict_
 template <typename T>
 __global__ void __launch_bounds__(kGenThreads)
 gen_stats_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd,
-                 const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld, int Hkv, int Lq, int Lk, int D, int W,
+                 const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs, int Hkv, int Lq, int Lk, int D, int W,
                  int g, int M, int mpad, float scale, int p_round, int y_round, float* __restrict__ ystat,
                  float* __restrict__ yf32, uint32_t* __restrict__ zero_ptr, int64_t zero_words) {
   __shared__ float qs[kGenMaxD];
@@ -64,14 +64,15 @@ gen_stats_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
   const T* qrow = q + (int64_t)b * q_sb + (int64_t)(hkv * g + gi) * q_sh + (int64_t)(Lq - W + w) * q_ss;
   for (int d = tid; d < D; d += kGenThreads) qs[d] = ld(qrow + (int64_t)d * q_sd);
   __syncthreads();
-  const T* kh = kp + (int64_t)head * kv_ld * D;
-  const T* vh = vp + (int64_t)head * kv_ld * D;
+  const T* kh = kp + b * kvs.k_sb + hkv * kvs.k_sh;
+  const T* vh = vp + b * kvs.v_sb + hkv * kvs.v_sh;
+  const int64_t k_sl = kvs.k_rb / sizeof(T), v_sl = kvs.v_rb / sizeof(T);
   const int bound = Lk - W + w;  // keys j <= bound are visible to this row
 
   // Sweep 1: maximum and sum of exp(l - max) per thread, then per row.
   float mt = -INFINITY, st = 0.f;
   for (int j = tid; j <= bound; j += kGenThreads) {
-    const float l = gen_logit(qs, kh + (int64_t)j * D, D, scale);
+    const float l = gen_logit(qs, kh + j * k_sl, D, scale);
     if (l > mt) {
       st = st * __expf(mt - l) + 1.f;
       mt = l;
@@ -100,7 +101,7 @@ gen_stats_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
     const int j = j0 + tid;
     float p = 0.f;
     if (j <= bound) {
-      p = fminf(__expf(gen_logit(qs, kh + (int64_t)j * D, D, scale) - lse), 1.f);
+      p = fminf(__expf(gen_logit(qs, kh + j * k_sl, D, scale) - lse), 1.f);
       if (p_round) p = round_through<T>(p);
     }
     __syncthreads();
@@ -109,7 +110,7 @@ gen_stats_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
     const int n = min(kGenThreads, bound + 1 - j0);
     for (int u = 0; u < n; ++u) {
       const float pu = ps[u];
-      const T* vr = vh + (int64_t)(j0 + u) * D;
+      const T* vr = vh + (j0 + u) * v_sl;
 #pragma unroll
       for (int c = 0; c < kGenCols; ++c)
         if (tid + c * kGenThreads < D) y[c] = fmaf(pu, ld(vr + tid + c * kGenThreads), y[c]);
@@ -128,7 +129,7 @@ gen_stats_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
 template <typename T, int R>
 __global__ void __launch_bounds__(kGenThreads)
 gen_score_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd,
-                 const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld, int Hkv, int Lq, int Lk, int D, int W,
+                 const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs, int Hkv, int Lq, int Lk, int D, int W,
                  int g, int M, int mpad, float scale, float eps, int p_round, const float* __restrict__ ystat,
                  const float* __restrict__ yf32, float* __restrict__ scores) {
   // R query rows of D, then R y rows of D (dynamic LDS).
@@ -141,8 +142,8 @@ gen_score_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
   const int head = blockIdx.x / tiles;
   const int j = (blockIdx.x % tiles) * kGenThreads + tid;
   const int b = head / Hkv, hkv = head % Hkv;
-  const T* krow = kp + ((int64_t)head * kv_ld + min(j, Lk - 1)) * D;
-  const T* vrow = vp + ((int64_t)head * kv_ld + min(j, Lk - 1)) * D;
+  const T* krow = kp + b * kvs.k_sb + hkv * kvs.k_sh + min(j, Lk - 1) * (int64_t)(kvs.k_rb / sizeof(T));
+  const T* vrow = vp + b * kvs.v_sb + hkv * kvs.v_sh + min(j, Lk - 1) * (int64_t)(kvs.v_rb / sizeof(T));
   float score = 0.f;
   for (int r0 = 0; r0 < M; r0 += R) {
     const int nr = min(R, M - r0);
@@ -189,21 +190,22 @@ gen_score_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
 
 template <typename T>
 static hipError_t launch_generic_t(const ScorePlan& p, int D, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss,
-                                   int64_t q_sd, const void* k, const void* v, int kv_ld, int Hkv, int Lq, int Lk,
+                                   int64_t q_sd, const KvSrc& kv, int Hkv, int Lq, int Lk,
                                    int W, float eps, int p_round, int y_round, float* scores, char* ws,
                                    uint32_t* zero_ptr, int64_t zero_words, hipStream_t st) {
   const float scale = 1.0f / sqrtf((float)D);
   float* ystat = reinterpret_cast<float*>(ws + p.off_stat);
   float* yf = reinterpret_cast<float*>(ws + p.off_yf);
   const T* qq = static_cast<const T*>(q);
-  const T* kk = static_cast<const T*>(k);
-  const T* vv = static_cast<const T*>(v);
+  const T* kk = static_cast<const T*>(kv.k);
+  const T* vv = static_cast<const T*>(kv.v);
+  const KvStride kvs = kv_strides(kv, sizeof(T));
   launch(gen_stats_kernel<T>, dim3(p.heads * p.M), dim3(kGenThreads), 0, st, qq, q_sb, q_sh, q_ss, q_sd, kk, vv,
-         kv_ld, Hkv, Lq, Lk, D, W, p.g, p.M, p.mpad, scale, p_round, y_round, ystat, yf, zero_ptr, zero_words);
+         kvs, Hkv, Lq, Lk, D, W, p.g, p.M, p.mpad, scale, p_round, y_round, ystat, yf, zero_ptr, zero_words);
   const int tiles = (Lk + kGenThreads - 1) / kGenThreads;
   const size_t lds = (size_t)2 * gen_rows(D) * D * sizeof(float);
   auto score = [&](auto kern) {
-    launch(kern, dim3(p.heads * tiles), dim3(kGenThreads), lds, st, qq, q_sb, q_sh, q_ss, q_sd, kk, vv, kv_ld, Hkv,
+    launch(kern, dim3(p.heads * tiles), dim3(kGenThreads), lds, st, qq, q_sb, q_sh, q_ss, q_sd, kk, vv, kvs, Hkv,
            Lq, Lk, D, W, p.g, p.M, p.mpad, scale, eps, p_round, ystat, yf, scores);
   };
   switch (gen_rows(D)) {
@@ -220,19 +222,19 @@ static hipError_t launch_generic_t(const ScorePlan& p, int D, const void* q, int
 int64_t generic_max_head_dim() { return kGenMaxD; }
 
 hipError_t launch_scores_generic(const ScorePlan& p, int dtype, int D, const void* q, int64_t q_sb, int64_t q_sh,
-                                 int64_t q_ss, int64_t q_sd, const void* k, const void* v, int kv_ld, int Hkv, int Lq,
+                                 int64_t q_ss, int64_t q_sd, const KvSrc& kv, int Hkv, int Lq,
                                  int Lk, int W, float eps, int p_round, int y_round, float* scores, char* ws,
                                  uint32_t* zero_ptr, int64_t zero_words, hipStream_t st) {
   if (D < 1 || D > kGenMaxD) return hipErrorInvalidValue;
   switch (dtype) {
     case kDtypeBf16:
-      return launch_generic_t<__bf16>(p, D, q, q_sb, q_sh, q_ss, q_sd, k, v, kv_ld, Hkv, Lq, Lk, W, eps, p_round,
+      return launch_generic_t<__bf16>(p, D, q, q_sb, q_sh, q_ss, q_sd, kv, Hkv, Lq, Lk, W, eps, p_round,
                                       y_round, scores, ws, zero_ptr, zero_words, st);
     case kDtypeFp16:
-      return launch_generic_t<_Float16>(p, D, q, q_sb, q_sh, q_ss, q_sd, k, v, kv_ld, Hkv, Lq, Lk, W, eps, p_round,
+      return launch_generic_t<_Float16>(p, D, q, q_sb, q_sh, q_ss, q_sd, kv, Hkv, Lq, Lk, W, eps, p_round,
                                         y_round, scores, ws, zero_ptr, zero_words, st);
     case kDtypeFp32:
-      return launch_generic_t<float>(p, D, q, q_sb, q_sh, q_ss, q_sd, k, v, kv_ld, Hkv, Lq, Lk, W, eps, p_round,
+      return launch_generic_t<float>(p, D, q, q_sb, q_sh, q_ss, q_sd, kv, Hkv, Lq, Lk, W, eps, p_round,
                                      y_round, scores, ws, zero_ptr, zero_words, st);
   }
   return hipErrorInvalidValue;

@@ -72,9 +72,20 @@ struct FuseSelect {
   const SelectCompact* cp;
   int* tail_done;
 };
-// K/V: [B*Hkv, kv_ld, D] with rows 0 .. Lk-1 of each head used (kv_ld = Lk: contiguous).
+// K/V [B, Hkv, Lk, D] by element strides (batch, head, row; D contiguous).
+struct KvSrc {
+  const void* k;
+  const void* v;
+  int64_t k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;
+};
+struct KvStride;  // the same for the kernels (dkv_common.h)
+KvStride kv_strides(const KvSrc& kv, int64_t elem_bytes);
+// Whether the scoring kernels' 32-bit row offsets reach every row of a head
+// (and the rows a tile loop asks for past its range) with rows this far
+// apart, and rows do not overlap.
+bool kv_rows_fit(int64_t row_stride, int64_t elem_bytes, int64_t Lk, int64_t D);
 hipError_t launch_scores(const ScorePlan& p, int dtype, int D, const void* q, int64_t q_sb, int64_t q_sh,
-                         int64_t q_ss, int64_t q_sd, const void* k, const void* v, int kv_ld, int Hkv, int Lq,
+                         int64_t q_ss, int64_t q_sd, const KvSrc& kv, int Hkv, int Lq,
                          int Lk, int W, float eps, int p_round, int y_round, float* scores, char* ws,
                          uint32_t* zero_ptr, int64_t zero_words, const FuseSelect* fuse, hipStream_t st);
 // Counters at the start of every score / evict workspace
@@ -86,7 +97,7 @@ hipError_t launch_debug_state(const ScorePlan& p, const char* ws, int D, float* 
 // The generic scoring kernels (fp32 arithmetic on the vector ALUs) on the
 // same plan's workspace; no fused pooling.
 hipError_t launch_scores_generic(const ScorePlan& p, int dtype, int D, const void* q, int64_t q_sb, int64_t q_sh,
-                                 int64_t q_ss, int64_t q_sd, const void* k, const void* v, int kv_ld, int Hkv, int Lq,
+                                 int64_t q_ss, int64_t q_sd, const KvSrc& kv, int Hkv, int Lq,
                                  int Lk, int W, float eps, int p_round, int y_round, float* scores, char* ws,
                                  uint32_t* zero_ptr, int64_t zero_words, hipStream_t st);
 int64_t generic_max_head_dim();
@@ -120,12 +131,10 @@ int64_t select_zero_words(int64_t rows);
 // Longest row the selection kernels take.
 int64_t select_max_len();
 // Optional K/V gather fused into the selection's emit stage: rows of
-// [B, H, L, D] sources (element strides s_b, s_h, s_l; D contiguous; 16-byte
-// aligned rows) go to contiguous [B, H, keep, D] outputs.
+// [B, H, L, D] sources (D contiguous; 16-byte aligned rows) go to contiguous [B, H, keep, D] outputs.
 struct SelectCompact {
-  const void* k;
-  const void* v;
-  int64_t s_b, s_h, s_l, elem_bytes, D;
+  KvSrc src;
+  int64_t elem_bytes, D;
   int H;
   void* k_out;
   void* v_out;

@@ -50,7 +50,7 @@ namespace dkv {
 template <typename T, int D, int WAVES, int MINW>
 __global__ void __launch_bounds__(64 * WAVES, MINW)
 pass1_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd, bool qvec,
-             const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld,
+             const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs,
              int Hkv, int Lq, int Lk, int W, int g, int M, int n_mc, int n_splits, int kps,
              float scale_log2, float* __restrict__ part_ml, float* __restrict__ part_y,
              int2* __restrict__ part_cand) {
@@ -95,19 +95,18 @@ pass1_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, 
 
   const int k_begin = split * kps;
   const int k_end = min(k_begin + kps, Lk);
-  const int64_t roff = ((int64_t)head * kv_ld + k_begin) * D;
-  const uint32_t range = (uint32_t)(k_end - k_begin) * (D * sizeof(T));
-  const rsrc_t krs = make_rsrc(kp + roff, range), vrs = make_rsrc(vp + roff, range);
-  const uint32_t k_lane = (li * D + 8 * lg) * sizeof(T);
+  const rsrc_t krs = head_rows<T, D>(kp + b * kvs.k_sb + hkv * kvs.k_sh, kvs.k_rb, k_begin, k_end);
+  const rsrc_t vrs = head_rows<T, D>(vp + b * kvs.v_sb + hkv * kvs.v_sh, kvs.v_rb, k_begin, k_end);
+  const uint32_t k_lane = li * kvs.k_rb + 8 * lg * sizeof(T);
   // V chunk i of a lane: row lane / CPR + i * GRP of the tile, columns
   // 8 (lane % CPR) .. +7.
-  const uint32_t v_lane = ((lane / CPR) * D + 8 * (lane % CPR)) * sizeof(T);
+  const uint32_t v_lane = (lane / CPR) * kvs.v_rb + 8 * (lane % CPR) * sizeof(T);
   const int v_row = lane / CPR, v_col = 8 * (lane % CPR);
   uint32_t* vt = lds + wv * kVTileWords;
   auto load_v = [&](u32x4 (&vc)[NVC], int t) __attribute__((always_inline)) {
-    const uint32_t base = v_lane + (uint32_t)t * (D * sizeof(T));
+    const uint32_t base = v_lane + (uint32_t)t * kvs.v_rb;
 #pragma unroll
-    for (int i = 0; i < NVC; ++i) vc[i] = buf_load16(vrs, base + (uint32_t)(i * GRP * D * sizeof(T)));
+    for (int i = 0; i < NVC; ++i) vc[i] = buf_load16(vrs, base + (uint32_t)(i * GRP) * kvs.v_rb);
   };
 
   float m2[kMB], lsum[kMB];
@@ -149,7 +148,7 @@ pass1_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, 
     // The K registers are free again: start the K loads of tile tn (zeros
     // past the range; unconditional, so that the compiler's wait counts stay
     // exact) before waiting for this tile's V.
-    load_rows_op<T, D>(kop, krs, k_lane, tn);
+    load_rows_op<T, D>(kop, krs, k_lane, tn, kvs.k_rb);
 
     // The V rows -> LDS, as loaded.
 #pragma unroll
@@ -197,7 +196,7 @@ pass1_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, 
   // order, and so every bit of the result, is the same on every call.
   const int nrel = k_end - k_begin;
   int t = wv * kTile;  // relative to k_begin
-  load_rows_op<T, D>(kop, krs, k_lane, t);  // zeros if t >= nrel
+  load_rows_op<T, D>(kop, krs, k_lane, t, kvs.k_rb);  // zeros if t >= nrel
   load_v(vch, t);
   for (; t < nrel; t += stride) tile(kop, vch, k_begin + t, t + stride);
 
@@ -305,7 +304,7 @@ constexpr int kWideWaves = 8;
 template <typename T, int D, int kWideG>
 __global__ void __launch_bounds__(64 * kWideWaves, 1)
 pass1w_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd, bool qvec,
-              const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld,
+              const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs,
               int Hkv, int Lq, int Lk, int W, int g, int M, int n_mc, int n_splits, int kps,
               float scale_log2, float* __restrict__ part_ml, float* __restrict__ part_y,
               int2* __restrict__ part_cand) {
@@ -349,22 +348,21 @@ pass1w_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss,
 
   const int k_begin = split * kps;
   const int k_end = min(k_begin + kps, Lk);
-  const int64_t roff = ((int64_t)head * kv_ld + k_begin) * D;
-  const uint32_t range = (uint32_t)(k_end - k_begin) * (D * sizeof(T));
-  const rsrc_t krs = make_rsrc(kp + roff, range), vrs = make_rsrc(vp + roff, range);
+  const rsrc_t krs = head_rows<T, D>(kp + b * kvs.k_sb + hkv * kvs.k_sh, kvs.k_rb, k_begin, k_end);
+  const rsrc_t vrs = head_rows<T, D>(vp + b * kvs.v_sb + hkv * kvs.v_sh, kvs.v_rb, k_begin, k_end);
   // This thread's share of a tile: chunk tid of K and of V (row tid / CPR,
   // chunk tid % CPR).
   const int kr = tid / CPR, kc = tid % CPR;
-  const uint32_t k_off = (uint32_t)(kr * D + 8 * kc) * sizeof(T);
+  const uint32_t k_off = kr * kvs.k_rb + 8 * kc * sizeof(T), v_off = kr * kvs.v_rb + 8 * kc * sizeof(T);
   u32x4 kreg[kWideG], vreg[kWideG];
   // Loads of tile group grp (rows past the range read as zeros).
   auto issue = [&](int grp) __attribute__((always_inline)) {
 #pragma unroll
     for (int gt = 0; gt < kWideG; ++gt) {
-      const uint32_t base = (uint32_t)((grp * kWideG + gt) * kTile) * (D * sizeof(T));
+      const uint32_t row = (uint32_t)((grp * kWideG + gt) * kTile);
       if (tid < KCH) {
-        kreg[gt] = buf_load16(krs, base + k_off);
-        vreg[gt] = buf_load16(vrs, base + k_off);
+        kreg[gt] = buf_load16(krs, row * kvs.k_rb + k_off);
+        vreg[gt] = buf_load16(vrs, row * kvs.v_rb + v_off);
       }
     }
   };
@@ -505,7 +503,7 @@ template <typename T, int D>
 __global__ void __launch_bounds__(64 * kMergeRows)
 merge_kernel(const float* __restrict__ part_ml, const float* __restrict__ part_y, const int2* __restrict__ part_cand,
              int n_mc, int n_splits, int M, int n_rows, int p_round, int y_round, const T* __restrict__ q,
-             int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd, const T* __restrict__ vp, int kv_ld, int Lk,
+             int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd, const T* __restrict__ vp, KvStride kvs, int Lk,
              int Hkv, int g, int W, int Lq, u32x4* __restrict__ opblk, float* __restrict__ stblk,
              float* __restrict__ ystat, float* __restrict__ yf32, uint32_t* __restrict__ zero_ptr,
              int64_t zero_words) {
@@ -526,7 +524,7 @@ merge_kernel(const float* __restrict__ part_ml, const float* __restrict__ part_y
   const int rid =
       __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, gridDim.x) * kMergeRows + (threadIdx.x >> 6));
   merge_row<T, D>(rid, part_ml, part_y, part_cand, n_mc, n_splits, M, n_rows, p_round, y_round, q, q_sb, q_sh,
-                  q_ss, q_sd, vp, kv_ld, Lk, Hkv, g, W, Lq, opblk, stblk, ystat, yf32);
+                  q_ss, q_sd, vp, kvs, Lk, Hkv, g, W, Lq, opblk, stblk, ystat, yf32);
   // Last, so that the argument loads it needs do not delay the row's first loads.
   if (zero_ptr)
     for (int64_t i = (int64_t)blockIdx.x * (64 * kMergeRows) + threadIdx.x; i < zero_words;
@@ -547,7 +545,7 @@ merge_kernel(const float* __restrict__ part_ml, const float* __restrict__ part_y
 
 template <typename T, int D, int WAVES, int MINW, bool PR>
 __global__ void __launch_bounds__(64 * WAVES, MINW)
-pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld,
+pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs,
              int Hkv, int Lq, int Lk, int W, int g, int M, int n_mc, int cg, int n_splits, int kps,
              float scale_log2, float eps, float small_c2,
              const u32x4* __restrict__ opblk, const float* __restrict__ stblk, float* __restrict__ scores,
@@ -569,7 +567,13 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld,
   DKV_ARG_NOW(stblk);
   DKV_ARG_NOW(n_splits);
   DKV_ARG_NOW(kps);
-  DKV_ARG_NOW(kv_ld);
+  DKV_ARG_NOW(Hkv);
+  DKV_ARG_NOW(kvs.k_sb);
+  DKV_ARG_NOW(kvs.k_sh);
+  DKV_ARG_NOW(kvs.v_sb);
+  DKV_ARG_NOW(kvs.v_sh);
+  DKV_ARG_NOW(kvs.k_rb);
+  DKV_ARG_NOW(kvs.v_rb);
   DKV_ARG_NOW(Lk);
   DKV_ARG_NOW(n_mc);
   DKV_ARG_NOW(cg);
@@ -577,6 +581,7 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld,
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
   const int split = lid % n_splits;
   const int head = lid / n_splits;
+  const int b = head / Hkv, hkv = head % Hkv;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4;
 
@@ -584,10 +589,9 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld,
   const float out_scale = -2.0f * (1.0f / static_cast<float>(g));
   const int k_begin = split * kps;
   const int k_end = min(k_begin + kps, Lk);
-  const int64_t roff = ((int64_t)head * kv_ld + k_begin) * D;
-  const uint32_t range = (uint32_t)(k_end - k_begin) * (D * sizeof(T));
-  const rsrc_t krs = make_rsrc(kp + roff, range), vrs = make_rsrc(vp + roff, range);
-  const uint32_t k_lane = (li * D + 8 * lg) * sizeof(T);
+  const rsrc_t krs = head_rows<T, D>(kp + b * kvs.k_sb + hkv * kvs.k_sh, kvs.k_rb, k_begin, k_end);
+  const rsrc_t vrs = head_rows<T, D>(vp + b * kvs.v_sb + hkv * kvs.v_sh, kvs.v_rb, k_begin, k_end);
+  const uint32_t k_lane = li * kvs.k_rb + 8 * lg * sizeof(T), v_lane = li * kvs.v_rb + 8 * lg * sizeof(T);
   const int ntiles = (k_end - k_begin + kTile - 1) / kTile;
   __shared__ uint32_t s_next;
   const int unmasked_end = Lk - W + 1;
@@ -618,8 +622,8 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld,
     // not depend on the assignment.
     const int tw = wv;
     __syncthreads();  // the previous group's LDS operands and s_next are dead
-    load_rows_op<T, D>(kop, krs, k_lane, tw * kTile);
-    load_rows_op<T, D>(vop, vrs, k_lane, tw * kTile);
+    load_rows_op<T, D>(kop, krs, k_lane, tw * kTile, kvs.k_rb);
+    load_rows_op<T, D>(vop, vrs, v_lane, tw * kTile, kvs.v_rb);
     if (threadIdx.x == 0) s_next = WAVES;
     // The pooling histogram, zeroed once the first loads are out.
     if (first && fz.enabled && fz.sc_lds)
@@ -689,7 +693,7 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld,
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) sacc[kb][mb] = Elem<T>::mfma(qo, kop[kb][kk], sacc[kb][mb]);
           }
-        if (refill) load_rows_op<T, D>(kop, krs, k_lane, tn);
+        if (refill) load_rows_op<T, D>(kop, krs, k_lane, tn, kvs.k_rb);
 #pragma unroll
         for (int mb = 0; mb < kMB; ++mb)
 #pragma unroll
@@ -702,7 +706,7 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld,
               gacc[kb][mb] = Elem<T>::mfma(yl, vop[kb][kk], gacc[kb][mb]);
             }
           }
-        if (refill) load_rows_op<T, D>(vop, vrs, k_lane, tn);
+        if (refill) load_rows_op<T, D>(vop, vrs, v_lane, tn, kvs.v_rb);
         // sc accumulates w * (-dist2/2).  The causal bound, and the direct
         // distance at a row's dominant key (merge), are applied only in
         // tiles that reach the bound or hold such a key (and with padding
@@ -836,7 +840,7 @@ __device__ __forceinline__ float sum_over_row_lanes(float x) {
 
 template <typename T, int D, int kG, bool PR>
 __global__ void __launch_bounds__(64 * kWideWaves, 1)
-pass2w_kernel(const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld, int Hkv, int Lq, int Lk, int W, int g,
+pass2w_kernel(const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs, int Hkv, int Lq, int Lk, int W, int g,
               int M, int n_mc, int n_splits, int kps, float scale_log2, float eps, float small_c2,
               const u32x4* __restrict__ opblk, const float* __restrict__ stblk, float* __restrict__ scores, SelFuse fz) {
   typedef typename Elem<T>::v8 v8;
@@ -872,9 +876,9 @@ pass2w_kernel(const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld, int
   const float out_scale = -2.0f * (1.0f / static_cast<float>(g));
   const int k_begin = split * kps;
   const int k_end = min(k_begin + kps, Lk);
-  const int64_t roff = ((int64_t)head * kv_ld + k_begin) * D;
-  const uint32_t range = (uint32_t)(k_end - k_begin) * RB;
-  const rsrc_t krs = make_rsrc(kp + roff, range), vrs = make_rsrc(vp + roff, range);
+  const int b = head / Hkv, hkv = head % Hkv;
+  const rsrc_t krs = head_rows<T, D>(kp + b * kvs.k_sb + hkv * kvs.k_sh, kvs.k_rb, k_begin, k_end);
+  const rsrc_t vrs = head_rows<T, D>(vp + b * kvs.v_sb + hkv * kvs.v_sh, kvs.v_rb, k_begin, k_end);
   const int nrel = k_end - k_begin;
   const int ntiles = (nrel + kTile - 1) / kTile;
   const int ngroups = (ntiles + kG - 1) / kG;
@@ -917,15 +921,15 @@ pass2w_kernel(const T* __restrict__ kp, const T* __restrict__ vp, int kv_ld, int
   // Staging: thread tid < KCH owns chunk tid % CPR of row tid / CPR of each
   // tile, of K and of V.
   const int sr = tid / CPR, scn = tid % CPR;
-  const uint32_t s_off = (uint32_t)(sr * D + 8 * scn) * sizeof(T);
+  const uint32_t k_off = sr * kvs.k_rb + 8 * scn * sizeof(T), v_off = sr * kvs.v_rb + 8 * scn * sizeof(T);
   u32x4 kreg[kG], vreg[kG];
   auto issue = [&](int grp) __attribute__((always_inline)) {
 #pragma unroll
     for (int gt = 0; gt < kG; ++gt) {
-      const uint32_t base = (uint32_t)((grp * kG + gt) * kTile) * RB;
+      const uint32_t row = (uint32_t)((grp * kG + gt) * kTile);
       if (tid < KCH) {
-        kreg[gt] = buf_load16(krs, base + s_off);
-        vreg[gt] = buf_load16(vrs, base + s_off);
+        kreg[gt] = buf_load16(krs, row * kvs.k_rb + k_off);
+        vreg[gt] = buf_load16(vrs, row * kvs.v_rb + v_off);
       }
     }
   };
@@ -1187,6 +1191,17 @@ ScorePlan make_score_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Lk, int64_
   return p;
 }
 
+bool kv_rows_fit(int64_t row_stride, int64_t elem_bytes, int64_t Lk, int64_t D) {
+  // The stream kernels ask for up to a few hundred rows past a split's end.
+  constexpr int64_t kPastEnd = 1024;
+  return row_stride >= D && row_stride <= (int64_t(1) << 31) / elem_bytes / (Lk + kPastEnd);
+}
+
+KvStride kv_strides(const KvSrc& kv, int64_t elem_bytes) {
+  return KvStride{kv.k_sb, kv.k_sh, kv.v_sb, kv.v_sh, (uint32_t)(kv.k_sl * elem_bytes),
+                  (uint32_t)(kv.v_sl * elem_bytes)};
+}
+
 namespace {
 // Process-wide settings of the selection tail, read once per call (relaxed:
 // a call in flight on another thread sees either the old or the new value).
@@ -1233,7 +1248,7 @@ void set_tail_select(int mode, int spin, int spin_b) {
 
 template <typename T, int D>
 static hipError_t launch_scores_t(const ScorePlan& p, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss,
-                                  int64_t q_sd, const void* k, const void* v, int kv_ld, int Hkv, int Lq, int Lk,
+                                  int64_t q_sd, const KvSrc& kv, int Hkv, int Lq, int Lk,
                                   int W, float eps, int p_round, int y_round, float* scores, char* ws,
                                   uint32_t* zero_ptr, int64_t zero_words, const FuseSelect* fuse, hipStream_t st) {
   const float scale_log2 = 1.4426950408889634f / sqrtf((float)D);
@@ -1249,27 +1264,28 @@ static hipError_t launch_scores_t(const ScorePlan& p, const void* q, int64_t q_s
   float* yf = reinterpret_cast<float*>(ws + p.off_yf);
   int2* part_cand = reinterpret_cast<int2*>(ws + p.off_cand);
   const T* qq = static_cast<const T*>(q);
-  const T* kk = static_cast<const T*>(k);
-  const T* vv = static_cast<const T*>(v);
+  const T* kk = static_cast<const T*>(kv.k);
+  const T* vv = static_cast<const T*>(kv.v);
+  const KvStride kvs = kv_strides(kv, sizeof(T));
 
   const bool qvec = q_sd == 1 && (q_sb % 8) == 0 && (q_sh % 8) == 0 && (q_ss % 8) == 0 &&
                     (reinterpret_cast<uintptr_t>(q) & 15u) == 0;
   const dim3 g1(p.heads * p.n_mc * p.s1);
   if (p.p1_wide) {
     launch((pass1w_kernel<T, D, DKV_P1_WIDE_GROUP>), dim3(p.heads * p.s1), dim3(64 * kWideWaves), 0, st, qq, q_sb,
-           q_sh, q_ss, q_sd, qvec, kk, vv, kv_ld, Hkv, Lq, Lk, W, p.g, p.M, p.n_mc, p.s1, p.kps1, scale_log2, part_ml,
+           q_sh, q_ss, q_sd, qvec, kk, vv, kvs, Hkv, Lq, Lk, W, p.g, p.M, p.n_mc, p.s1, p.kps1, scale_log2, part_ml,
            part_y, part_cand);
   } else if (p.p1_waves == 8) {
-    launch((pass1_kernel<T, D, 8, 1>), g1, dim3(512), 0, st, qq, q_sb, q_sh, q_ss, q_sd, qvec, kk, vv, kv_ld, Hkv,
+    launch((pass1_kernel<T, D, 8, 1>), g1, dim3(512), 0, st, qq, q_sb, q_sh, q_ss, q_sd, qvec, kk, vv, kvs, Hkv,
            Lq, Lk, W, p.g, p.M, p.n_mc, p.s1, p.kps1, scale_log2, part_ml, part_y, part_cand);
   } else {
-    launch((pass1_kernel<T, D, 4, 1>), g1, dim3(256), 0, st, qq, q_sb, q_sh, q_ss, q_sd, qvec, kk, vv, kv_ld, Hkv,
+    launch((pass1_kernel<T, D, 4, 1>), g1, dim3(256), 0, st, qq, q_sb, q_sh, q_ss, q_sd, qvec, kk, vv, kvs, Hkv,
            Lq, Lk, W, p.g, p.M, p.n_mc, p.s1, p.kps1, scale_log2, part_ml, part_y, part_cand);
   }
   const int n_rows = p.heads * p.mpad;
   launch((merge_kernel<T, D>), dim3((n_rows + kMergeRows - 1) / kMergeRows), dim3(64 * kMergeRows), 0, st,
                      part_ml, part_y, part_cand, p.n_mc, p.s1, p.M, n_rows, p_round, y_round, qq, q_sb, q_sh, q_ss,
-                     q_sd, vv, kv_ld, Lk, Hkv, p.g, W, Lq, opblk, stblk, ystat, yf, zero_ptr, zero_words);
+                     q_sd, vv, kvs, Lk, Hkv, p.g, W, Lq, opblk, stblk, ystat, yf, zero_ptr, zero_words);
   // Named here, right after merge, so that the compiler lays pass 2's code
   // out next to pass 1's and merge's: the three run back to back, and their
   // code shares each CU pair's instruction cache.
@@ -1295,10 +1311,10 @@ static hipError_t launch_scores_t(const ScorePlan& p, const void* q, int64_t q_s
   if (p.p1_wide) {
     // One sweep over K/V for all row-chunks (pass2w); its LDS is static.
     if (p_round)
-      launch((pass2w_kernel<T, D, DKV_P2_WIDE_GROUP, true>), g2, dim3(64 * kWideWaves), 0, st, kk, vv, kv_ld, Hkv, Lq,
+      launch((pass2w_kernel<T, D, DKV_P2_WIDE_GROUP, true>), g2, dim3(64 * kWideWaves), 0, st, kk, vv, kvs, Hkv, Lq,
              Lk, W, p.g, p.M, p.n_mc, p.s2, p.kps2, scale_log2, eps, small_c2, opblk, stblk, scores, fz);
     else
-      launch((pass2w_kernel<T, D, DKV_P2_WIDE_GROUP, false>), g2, dim3(64 * kWideWaves), 0, st, kk, vv, kv_ld, Hkv,
+      launch((pass2w_kernel<T, D, DKV_P2_WIDE_GROUP, false>), g2, dim3(64 * kWideWaves), 0, st, kk, vv, kvs, Hkv,
              Lq, Lk, W, p.g, p.M, p.n_mc, p.s2, p.kps2, scale_log2, eps, small_c2, opblk, stblk, scores, fz);
     return hipGetLastError();
   }
@@ -1319,22 +1335,22 @@ static hipError_t launch_scores_t(const ScorePlan& p, const void* q, int64_t q_s
       if (fuse->tail_done) *fuse->tail_done = 1;
     }
   }
-  launch(k2, g2, dim3(512), lds2, st, kk, vv, kv_ld, Hkv, Lq, Lk, W, p.g, p.M, p.n_mc, cg, p.s2, p.kps2, scale_log2,
+  launch(k2, g2, dim3(512), lds2, st, kk, vv, kvs, Hkv, Lq, Lk, W, p.g, p.M, p.n_mc, cg, p.s2, p.kps2, scale_log2,
          eps, small_c2, opblk, stblk, scores, fz);
   return hipGetLastError();
 }
 
 hipError_t launch_scores(const ScorePlan& p, int dtype, int D, const void* q, int64_t q_sb, int64_t q_sh,
-                         int64_t q_ss, int64_t q_sd, const void* k, const void* v, int kv_ld, int Hkv, int Lq,
+                         int64_t q_ss, int64_t q_sd, const KvSrc& kv, int Hkv, int Lq,
                          int Lk, int W, float eps, int p_round, int y_round, float* scores, char* ws,
                          uint32_t* zero_ptr, int64_t zero_words, const FuseSelect* fuse, hipStream_t st) {
   if (scores_generic(dtype, D, p.M)) {
     if (fuse) return hipErrorInvalidValue;  // the generic kernels have no pooling tail
-    return launch_scores_generic(p, dtype, D, q, q_sb, q_sh, q_ss, q_sd, k, v, kv_ld, Hkv, Lq, Lk, W, eps, p_round,
+    return launch_scores_generic(p, dtype, D, q, q_sb, q_sh, q_ss, q_sd, kv, Hkv, Lq, Lk, W, eps, p_round,
                                  y_round, scores, ws, zero_ptr, zero_words, st);
   }
 #define DKV_CASE(TT, DD)                                                                                   \
-  return launch_scores_t<TT, DD>(p, q, q_sb, q_sh, q_ss, q_sd, k, v, kv_ld, Hkv, Lq, Lk, W, eps, p_round, \
+  return launch_scores_t<TT, DD>(p, q, q_sb, q_sh, q_ss, q_sd, kv, Hkv, Lq, Lk, W, eps, p_round, \
                                  y_round, scores, ws, zero_ptr, zero_words, fuse, st)
   if (dtype == kDtypeBf16) {
     if (D == 32) DKV_CASE(__bf16, 32);

@@ -253,18 +253,25 @@ __device__ __forceinline__ void merge_wave_cands(const float* sm_cs, const int* 
 // Offsets are bytes relative to row k_begin; per-lane parts are computed once
 // and the tile offset is one add.
 // ---------------------------------------------------------------------------
-// 32 key rows as an MFMA A operand: lane (li, lg) holds row t+16kb+li,
-// head-dim columns 32kk+8lg .. +7.  `lane_off` = (li*D + 8*lg) * sizeof(T).
+// The view of rows [k_begin, k_end) of the head whose row 0 is at `head`.
+template <typename T, int D>
+__device__ __forceinline__ rsrc_t head_rows(const T* head, uint32_t rb, int k_begin, int k_end) {
+  return make_rsrc(reinterpret_cast<const char*>(head) + (int64_t)k_begin * rb,
+                   rows_bytes(k_end - k_begin, rb, D * sizeof(T)));
+}
+
+// 32 key rows, rb bytes apart, as an MFMA A operand: lane (li, lg) holds row
+// t+16kb+li, head-dim columns 32kk+8lg .. +7.  `lane_off` = li*rb + 8*lg*sizeof(T).
 template <typename T, int D>
 __device__ __forceinline__ void load_rows_op(typename Elem<T>::v8 (&op)[2][D / 32], rsrc_t rs, uint32_t lane_off,
-                                             int t) {
+                                             int t, uint32_t rb) {
   typedef typename Elem<T>::v8 v8;
-  const uint32_t base = lane_off + (uint32_t)t * (D * sizeof(T));
+  const uint32_t base = lane_off + (uint32_t)t * rb;
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
     for (int kk = 0; kk < D / 32; ++kk)
-      op[kb][kk] = bitcast_u4<v8>(buf_load16(rs, base + (16 * kb * D + 32 * kk) * sizeof(T)));
+      op[kb][kk] = bitcast_u4<v8>(buf_load16(rs, base + 16 * kb * rb + 32 * kk * (uint32_t)sizeof(T)));
 }
 
 template <typename T>
@@ -304,8 +311,8 @@ __device__ __forceinline__ void merge_row(int rid, const float* __restrict__ par
                                           const int2* __restrict__ part_cand, int n_mc, int n_splits, int M,
                                           int n_rows, int p_round, int y_round, const T* __restrict__ q,
                                           int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd,
-                                          const T* __restrict__ vp, int kv_ld, int Lk, int Hkv, int g, int W, int Lq,
-                                          u32x4* __restrict__ opblk, float* __restrict__ stblk,
+                                          const T* __restrict__ vp, const KvStride& kvs, int Lk, int Hkv, int g, int W,
+                                          int Lq, u32x4* __restrict__ opblk, float* __restrict__ stblk,
                                           float* __restrict__ ystat, float* __restrict__ yf32) {
   constexpr int DPL = D >= 64 ? D / 64 : 1;  // columns per lane (D = 32: lanes 32..63 hold none)
   constexpr int KK = D / 32;
@@ -447,11 +454,12 @@ __device__ __forceinline__ void merge_row(int rid, const float* __restrict__ par
     }
     // Their value rows, all loads unconditional (a row of no candidate reads
     // past the view: zeros, no memory request).
-    const rsrc_t rv = make_rsrc(vp + (int64_t)head * kv_ld * D, (uint32_t)Lk * D * sizeof(T));
+    const uint32_t v_end = rows_bytes(Lk, kvs.v_rb, D * sizeof(T));
+    const rsrc_t rv = make_rsrc(vp + (head / Hkv) * kvs.v_sb + (head % Hkv) * kvs.v_sh, v_end);
 #pragma unroll
     for (int u = 0; u < kCorrKeys; ++u) {
       const uint32_t off =
-          ck[u] >= 0 && col ? ((uint32_t)ck[u] * D + d0) * sizeof(T) : (uint32_t)Lk * D * sizeof(T);
+          ck[u] >= 0 && col ? (uint32_t)ck[u] * kvs.v_rb + d0 * (uint32_t)sizeof(T) : v_end;
       if constexpr (DPL == 1) {
         vb[u][0] = static_cast<float>(__builtin_bit_cast(T, buf_load2(rv, off)));
       } else {

@@ -463,8 +463,8 @@ sel_emit_kernel(int Lk, int window, int keep, int chunks, SelWs ws, int64_t* __r
     const int nk = (int)min(last - start, (uint32_t)kChunk);
     const int b = row / ca.H, h = row % ca.H;
     const int total = nk * ca.units;
-    const uint8_t* kb = ca.k + b * ca.sb + h * ca.sh;
-    const uint8_t* vb = ca.v + b * ca.sb + h * ca.sh;
+    const uint8_t* kb = ca.k + b * ca.k_sb + h * ca.k_sh;
+    const uint8_t* vb = ca.v + b * ca.v_sb + h * ca.v_sh;
     constexpr int kG = 8;  // 16-byte units of K and of V in flight per thread
     for (int t0 = tid; t0 < total; t0 += kG * kEmitT) {
       u32x4 kv[kG], vv[kG];
@@ -472,9 +472,9 @@ sel_emit_kernel(int Lk, int window, int keep, int chunks, SelWs ws, int64_t* __r
       for (int q = 0; q < kG; ++q) {
         const int t = t0 + q * kEmitT;
         if (t < total) {
-          const int64_t o = (int64_t)s_src[t / ca.units] * ca.sl + 16 * (t % ca.units);
-          kv[q] = *reinterpret_cast<const u32x4*>(kb + o);
-          vv[q] = *reinterpret_cast<const u32x4*>(vb + o);
+          const int64_t j = s_src[t / ca.units], u = 16 * (t % ca.units);
+          kv[q] = *reinterpret_cast<const u32x4*>(kb + j * ca.k_sl + u);
+          vv[q] = *reinterpret_cast<const u32x4*>(vb + j * ca.v_sl + u);
         }
       }
 #pragma unroll
@@ -506,11 +506,14 @@ int64_t select_max_len() { return (int64_t)kMaxChunks * kChunk; }
 CompactArgs compact_args(const SelectCompact* cp) {
   CompactArgs ca{};
   if (cp) {
-    ca.k = static_cast<const uint8_t*>(cp->k);
-    ca.v = static_cast<const uint8_t*>(cp->v);
-    ca.sb = cp->s_b * cp->elem_bytes;
-    ca.sh = cp->s_h * cp->elem_bytes;
-    ca.sl = cp->s_l * cp->elem_bytes;
+    ca.k = static_cast<const uint8_t*>(cp->src.k);
+    ca.v = static_cast<const uint8_t*>(cp->src.v);
+    ca.k_sb = cp->src.k_sb * cp->elem_bytes;
+    ca.k_sh = cp->src.k_sh * cp->elem_bytes;
+    ca.k_sl = cp->src.k_sl * cp->elem_bytes;
+    ca.v_sb = cp->src.v_sb * cp->elem_bytes;
+    ca.v_sh = cp->src.v_sh * cp->elem_bytes;
+    ca.v_sl = cp->src.v_sl * cp->elem_bytes;
     ca.H = cp->H;
     ca.units = (int)(cp->D * cp->elem_bytes / 16);
     ca.ko = static_cast<uint8_t*>(cp->k_out);

@@ -102,7 +102,7 @@ __device__ __forceinline__ uint32_t pooled_key(uint32_t bits, int j, int prot, u
 struct CompactArgs {
   const uint8_t* k;
   const uint8_t* v;
-  int64_t sb, sh, sl;  // source byte strides
+  int64_t k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;  // source byte strides
   int H;
   int units;           // 16-byte units per row
   uint8_t* ko;

@@ -168,8 +168,8 @@ __device__ __forceinline__ void tail_gather(const CompactArgs& ca, int row, int 
                                             const int* s_dst) {
   const int b = row / ca.H, hh = row % ca.H;
   const int total = nk * ca.units;
-  const uint8_t* kb = ca.k + b * ca.sb + hh * ca.sh;
-  const uint8_t* vb = ca.v + b * ca.sb + hh * ca.sh;
+  const uint8_t* kb = ca.k + b * ca.k_sb + hh * ca.k_sh;
+  const uint8_t* vb = ca.v + b * ca.v_sb + hh * ca.v_sh;
   constexpr int kG = 4;  // 16-byte units of K and of V in flight per thread
   for (int t0 = threadIdx.x; t0 < total; t0 += kG * NT) {
     u32x4 kv[kG], vv[kG];
@@ -177,9 +177,9 @@ __device__ __forceinline__ void tail_gather(const CompactArgs& ca, int row, int 
     for (int q = 0; q < kG; ++q) {
       const int t = t0 + q * NT;
       if (t < total) {
-        const int64_t o = (int64_t)s_src[t / ca.units] * ca.sl + 16 * (t % ca.units);
-        kv[q] = *reinterpret_cast<const u32x4*>(kb + o);
-        vv[q] = *reinterpret_cast<const u32x4*>(vb + o);
+        const int64_t j = s_src[t / ca.units], u = 16 * (t % ca.units);
+        kv[q] = *reinterpret_cast<const u32x4*>(kb + j * ca.k_sl + u);
+        vv[q] = *reinterpret_cast<const u32x4*>(vb + j * ca.v_sl + u);
       }
     }
 #pragma unroll
@@ -529,16 +529,16 @@ __device__ void fused_tail(const SelFuse& fz, const float* __restrict__ sc, uint
   const int units = ca.units;
   const int pre_rows = min((int)np_all, kPre * NT / units);
   const int bb = row / ca.H, hh = row % ca.H;
-  const uint8_t* kbase = ca.k + bb * ca.sb + hh * ca.sh;
-  const uint8_t* vbase = ca.v + bb * ca.sb + hh * ca.sh;
+  const uint8_t* kbase = ca.k + bb * ca.k_sb + hh * ca.k_sh;
+  const uint8_t* vbase = ca.v + bb * ca.v_sb + hh * ca.v_sh;
   u32x4 kpre[kPre], vpre[kPre];
 #pragma unroll
   for (int q = 0; q < kPre; ++q) {
     const int u = tid + q * NT;
     if (u < pre_rows * units) {
-      const int64_t o = (int64_t)s_pot[u / units] * ca.sl + 16 * (u % units);
-      kpre[q] = *reinterpret_cast<const u32x4*>(kbase + o);
-      vpre[q] = *reinterpret_cast<const u32x4*>(vbase + o);
+      const int64_t j = s_pot[u / units], c = 16 * (u % units);
+      kpre[q] = *reinterpret_cast<const u32x4*>(kbase + j * ca.k_sl + c);
+      vpre[q] = *reinterpret_cast<const u32x4*>(vbase + j * ca.v_sl + c);
     }
   }
   if (tid == 0) {
@@ -730,10 +730,10 @@ __device__ void fused_tail(const SelFuse& fz, const float* __restrict__ sc, uint
     const int j = s_pot[u / units];
     const int p = pos_of[j - k_begin];
     if (p >= 0) {
-      const int64_t os = (int64_t)j * ca.sl + 16 * (u % units);
+      const int64_t c = 16 * (u % units);
       const int64_t o = (orow + p) * units * 16 + 16 * (u % units);
-      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(kbase + os), reinterpret_cast<u32x4*>(ca.ko + o));
-      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(vbase + os), reinterpret_cast<u32x4*>(ca.vo + o));
+      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(kbase + j * ca.k_sl + c), reinterpret_cast<u32x4*>(ca.ko + o));
+      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(vbase + j * ca.v_sl + c), reinterpret_cast<u32x4*>(ca.vo + o));
     }
   }
 }

@@ -52,12 +52,10 @@ def _evict(query_states: torch.Tensor, key_states: torch.Tensor, value_states: t
     the current stream's shared one, so consecutive layers allocate no
     workspace.
     """
-    key_states = key_states.contiguous()
-    value_states = value_states.contiguous()
     fast = False
     if use_triton:
         try:
-            check_scoring_inputs(query_states, key_states, value_states, window_size)
+            check_scoring_inputs(query_states, key_states, value_states, window_size, require_contiguous=False)
             fast = True
         except AssertionError:
             fast = False

@@ -83,6 +83,24 @@ def _kv_operand(t: torch.Tensor) -> torch.Tensor:
     return t
 
 
+def _evict_kv(t: torch.Tensor):
+    """``t`` (K or V, [B, H, L, D]) as the layer-call reads it, and its
+    (batch, head, row) element strides: in place where its rows are whole
+    16-byte units apart and do not overlap (a decoder layer's [B, L, H, D]
+    projection seen as [B, H, L, D], say), else a dense copy.  The rule is
+    that of ``dropkv_evict_strided``."""
+    B, H, L, D = t.shape
+    dense = (H * L * D, L * D, D)
+    if t.is_contiguous():
+        return (t if _aligned(t) else t.clone()), dense
+    sb, sh, sl, sd = t.stride()
+    es = t.element_size()
+    if (sd == 1 and sl >= D and ((sb | sh | sl | D) * es) % 16 == 0 and _aligned(t)
+            and sl <= (1 << 31) // es // (L + 1024)):
+        return t, (sb, sh, sl)
+    return t.contiguous(), dense
+
+
 def _check_device(*ts: torch.Tensor) -> torch.device:
     dev = ts[0].device
     if dev.type != "cuda":
@@ -266,18 +284,19 @@ def evict(Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor, window: int, kernel
         raise RuntimeError("K and V must have the same shape")
     B, Hq, Lq, D = Q.shape
     Hkv, Lk = K.shape[1], K.shape[2]
-    K = _kv_operand(K)
-    V = _kv_operand(V)
+    K, k_strides = _evict_kv(K)
+    V, v_strides = _evict_kv(V)
     lib = _lib.load()
     ws = _stream_workspace(lib.dropkv_evict_workspace_bytes(B, Hq, Hkv, Lk, D, window, splits), dev)
     idx = torch.empty(B, Hkv, keep, dtype=torch.int64, device=dev)
-    ko = torch.empty(B, Hkv, keep, D, dtype=K.dtype, device=dev)
+    ko = torch.empty(B, Hkv, keep, D, dtype=Q.dtype, device=dev)
     vo = torch.empty_like(ko)
     pw = window if protect_window is None else protect_window
-    rc = lib.dropkv_evict(Q.data_ptr(), *Q.stride(), K.data_ptr(), V.data_ptr(), _DTYPE_CODE[Q.dtype],
-                          B, Hq, Hkv, Lq, Lk, D, int(window), float(eps), int(bool(p_round)), int(bool(y_round)),
-                          int(splits), int(kernel_size), int(pw), int(keep), None, idx.data_ptr(), ko.data_ptr(),
-                          vo.data_ptr(), ws.data_ptr(), ws.numel(), _stream(dev))
+    rc = lib.dropkv_evict_strided(Q.data_ptr(), *Q.stride(), K.data_ptr(), *k_strides, V.data_ptr(), *v_strides,
+                                  _DTYPE_CODE[Q.dtype], B, Hq, Hkv, Lq, Lk, D, int(window), float(eps),
+                                  int(bool(p_round)), int(bool(y_round)), int(splits), int(kernel_size), int(pw),
+                                  int(keep), None, idx.data_ptr(), ko.data_ptr(), vo.data_ptr(), int(keep),
+                                  ws.data_ptr(), ws.numel(), _stream(dev))
     _lib.check(rc, "dropkv_evict")
     return idx, ko, vo
 
@@ -323,14 +342,14 @@ class EvictPlan:
             raise RuntimeError("input shapes differ from the plan")
         if Q.dtype != self.dtype or K.dtype != self.dtype or V.dtype != self.dtype:
             raise RuntimeError("input dtype differs from the plan")
-        K = _kv_operand(K)
-        V = _kv_operand(V)
-        rc = _lib.load().dropkv_evict(
-            Q.data_ptr(), *Q.stride(), K.data_ptr(), V.data_ptr(), _DTYPE_CODE[self.dtype],
+        K, k_strides = _evict_kv(K)
+        V, v_strides = _evict_kv(V)
+        rc = _lib.load().dropkv_evict_strided(
+            Q.data_ptr(), *Q.stride(), K.data_ptr(), *k_strides, V.data_ptr(), *v_strides, _DTYPE_CODE[self.dtype],
             B, Hq, Hkv, Lq, Lk, D, self.window, self.eps, self.p_round, self.y_round, self.splits,
             self.kernel_size, self.protect_window, self.keep,
             self.scores.data_ptr() if self.scores is not None else None, self.keep_idx.data_ptr(),
-            self.k_out.data_ptr(), self.v_out.data_ptr(), self.ws.data_ptr(), self.ws.numel(),
+            self.k_out.data_ptr(), self.v_out.data_ptr(), self.keep, self.ws.data_ptr(), self.ws.numel(),
             _stream(self.dev))
         _lib.check(rc, "dropkv_evict")
         return self.keep_idx, self.k_out, self.v_out

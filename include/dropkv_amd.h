@@ -210,6 +210,22 @@ int dropkv_evict_noalloc(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss
  * buffers must not overlap the inputs.  With kv_ld = Lk and out_ld = keep it
  * is dropkv_evict.
  * ------------------------------------------------------------------------ */
+/* dropkv_evict_strided: dropkv_evict_ld on K/V of any layout with the D axis
+ * contiguous: row l of (batch b, KV head h) starts at element b*k_sb + h*k_sh +
+ * l*k_sl of k (v likewise), so that the [B, L, H, D] projections of a decoder
+ * layer are read in place.  Strides of anything but dense [B,Hkv,Lk,D] K/V
+ * must be whole 16-byte units, rows at least D elements apart, a head's rows
+ * (with 1024 more) within 2 GiB, D a whole number of 16-byte units and the
+ * outputs 16-byte aligned; otherwise DROPKV_E_UNSUPPORTED. */
+int dropkv_evict_strided(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd,
+                         const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sl,
+                         const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl, int dtype,
+                         int64_t B, int64_t Hq, int64_t Hkv, int64_t Lq, int64_t Lk, int64_t D,
+                         int64_t W, float eps, int p_round, int y_round, int64_t splits,
+                         int64_t kernel_size, int64_t protect_window, int64_t keep,
+                         float* scores, int64_t* keep_idx, void* k_out, void* v_out, int64_t out_ld,
+                         void* workspace, size_t workspace_bytes, void* stream);
+
 int dropkv_append(const void* k, const void* v, int64_t s_b, int64_t s_h, int64_t s_l, int64_t elem_bytes,
                   int64_t B, int64_t H, int64_t L, int64_t D, void* k_dst, void* v_dst, int64_t dst_ld,
                   int64_t row0, void* stream);
