@@ -1,8 +1,8 @@
-// DropKV scoring for the inputs the matrix-core kernels do not take: fp32
-// Q/K/V (the reference's deployed path scores them in PyTorch fp32,
-// dropkv_cache.py:399-460), or a head dimension outside the matrix-core set
-// (dropkv_scores_triton accepts any power of two >= 32,
-// dropkv_triton.py:707-713; the deployed path any D).
+// DropKV scoring for the inputs no matrix-core kernel takes: head dimensions
+// above 256, or whose rows are no whole 16-byte units (the deployed path of the
+// reference scores any D, dropkv_cache.py:399-460; dropkv_scores_triton any
+// power of two >= 32, dropkv_triton.py:707-713).  fp32 inputs and other head
+// dimensions go to dkv_generic_mfma.hip.
 //
 // Plain fp32 arithmetic on the vector ALUs, with the reference's semantics
 // computed exactly rather than corrected afterwards:
@@ -226,6 +226,9 @@ hipError_t launch_scores_generic(const ScorePlan& p, int dtype, int D, const voi
                                  int Lk, int W, float eps, int p_round, int y_round, float* scores, char* ws,
                                  uint32_t* zero_ptr, int64_t zero_words, hipStream_t st) {
   if (D < 1 || D > kGenMaxD) return hipErrorInvalidValue;
+  if (generic_on_mfma(dtype, D, Lk, kv))
+    return launch_scores_generic_mfma(p, dtype, D, q, q_sb, q_sh, q_ss, q_sd, kv, Hkv, Lq, Lk, W, eps, p_round,
+                                      y_round, scores, ws, zero_ptr, zero_words, st);
   switch (dtype) {
     case kDtypeBf16:
       return launch_generic_t<__bf16>(p, D, q, q_sb, q_sh, q_ss, q_sd, kv, Hkv, Lq, Lk, W, eps, p_round,

@@ -29,8 +29,9 @@ inline void launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, uint32_t shm
 // Element types (the DROPKV_BF16 / _FP16 / _FP32 codes of the C ABI).
 constexpr int kDtypeBf16 = 1, kDtypeFp16 = 2, kDtypeFp32 = 3;
 
-// Head dimensions of the matrix-core scoring kernels; every other one (and
-// fp32 inputs) takes the generic kernels (dkv_generic.hip).
+// Head dimensions of the tuned scoring pipeline (dkv_score.hip); every other
+// one (and fp32 inputs) takes the generic kernels (dkv_generic_mfma.hip up to
+// 256 columns, dkv_generic.hip).
 constexpr int64_t kMfmaHeadDims[] = {32, 64, 128};
 inline bool mfma_head_dim(int64_t D) {
   for (int64_t d : kMfmaHeadDims)
@@ -94,12 +95,18 @@ hipError_t launch_scores(const ScorePlan& p, int dtype, int D, const void* q, in
 constexpr size_t kSyncBytes = 4096;
 hipError_t launch_debug_state(const ScorePlan& p, const char* ws, int D, float* lse_out, float* y_out,
                               hipStream_t st);
-// The generic scoring kernels (fp32 arithmetic on the vector ALUs) on the
-// same plan's workspace; no fused pooling.
+// The generic scoring kernels on the same plan's workspace; no fused pooling.
 hipError_t launch_scores_generic(const ScorePlan& p, int dtype, int D, const void* q, int64_t q_sb, int64_t q_sh,
                                  int64_t q_ss, int64_t q_sd, const KvSrc& kv, int Hkv, int Lq,
                                  int Lk, int W, float eps, int p_round, int y_round, float* scores, char* ws,
                                  uint32_t* zero_ptr, int64_t zero_words, hipStream_t st);
+// Those of dkv_generic_mfma.hip, on the matrix cores, where generic_on_mfma
+// says that they take the call.
+bool generic_on_mfma(int dtype, int64_t D, int64_t Lk, const KvSrc& kv);
+hipError_t launch_scores_generic_mfma(const ScorePlan& p, int dtype, int D, const void* q, int64_t q_sb, int64_t q_sh,
+                                      int64_t q_ss, int64_t q_sd, const KvSrc& kv, int Hkv, int Lq, int Lk, int W,
+                                      float eps, int p_round, int y_round, float* scores, char* ws,
+                                      uint32_t* zero_ptr, int64_t zero_words, hipStream_t st);
 int64_t generic_max_head_dim();
 hipError_t launch_mfma_selftest(float* out, hipStream_t st);
 
