@@ -22,7 +22,6 @@
 namespace dkv {
 
 constexpr int kDecMaxG = 16;      // query heads per KV head: the 16 columns of the MFMA tiles
-constexpr int kDecStep = 64;      // keys per step of a split
 constexpr int kDecMaxSplits = 64;
 
 struct DecodeArgs {
@@ -35,7 +34,8 @@ struct DecodeArgs {
   void* vbuf;
   const int* n_rows;  // rows already stored (device)
   int B, Hq, Hkv, D, C, S;
-  int kps;  // rows of the buffer per split: ceil(C / S)
+  int kps;  // rows of the buffer per split (whole tiles)
+  int qvec, nvec;  // rows of q / of the new K and V as 16-byte loads
   float scale_log2;
   float* part_m;  // [B*Hkv, S, g]
   float* part_l;
@@ -45,59 +45,81 @@ struct DecodeArgs {
 };
 
 // One wave per (b, kv head, key split).  Split s owns buffer rows
-// [s * kps, (s + 1) * kps) whatever the row count, so its first step's loads
+// [s * kps, (s + 1) * kps) whatever the row count, so its first tile's loads
 // are issued before the count has arrived; rows past the new row n are
-// masked (splits past n write empty partials).  The new row is loaded into
-// registers with the first step, put into LDS in place of row n, and stored
-// into the buffer only after the attention, so that no wave waits on it.
-// Each step covers 64 keys: their K and V rows (contiguous in the cache
-// buffer) are copied to LDS with 16-byte LDS-DMA loads (buffer view of the
-// head's rows: rows past the buffer read as zeros).  Both products run on
-// the matrix cores with the group's query heads as the 16 columns (heads
-// past the group are zero): S^T = K Q^T per 16-key block, and
-// O^T += V^T P^T per 32 keys, V read transposed from LDS and P in two parts
-// (hi and the rounded remainder, ~16 significant bits).  Lane (li, lg) holds
-// head li's logits of keys 16 kb + 4 lg + r and its outputs at columns
-// 16 dt + 4 lg + r; a head's maximum and sum combine its four lanes.
-typedef __attribute__((address_space(3))) void lds_void_t;
+// masked (splits past n write empty partials).  The new row is held in
+// registers, takes row n's place in its tile, and is stored into the buffer
+// only after the attention, so that no wave waits on it.  Tiles of 32 keys
+// (buffer views: rows past the buffer read as zeros): K in registers as the
+// MFMA operand, V through LDS for the transposing reads, and the next tile's
+// loads issued as soon as a tile's registers are consumed, so that a wave
+// always has 16 KB on the way (D = 128).  Both products run on the matrix
+// cores with the group's query heads as the 16 columns (heads past the group
+// are zero): S^T = K Q^T per 16-key block, and O^T += V^T P^T per 32 keys, P in
+// two parts (hi and the rounded remainder, ~16 significant bits).  Lane
+// (li, lg) holds head li's logits of keys 16 kb + 4 lg + r and its outputs at
+// columns 16 dt + 4 lg + r; a head's maximum and sum combine its four lanes.
+//
+// Bound: HBM for long caches of a batch.  With 64-key steps staged through LDS
+// one after the other (32 KB a wave, five waves per CU, nothing in flight
+// during a step's arithmetic, last steps of a few rows) a call with 8 x 8 heads
+// of 8004 rows, D = 128 (262 MB), took 75.6 us; tiles in flight under the
+// arithmetic, whole tiles per split: 50 us (5.2 TB/s).
+constexpr int kDecTile = 32;
+
+// Eight elements from d0 of a row: one 16-byte load, or by stride.
+template <typename T>
+__device__ __forceinline__ typename Elem<T>::v8 load8(const T* row, int d0, int64_t sd, bool vec) {
+  typename Elem<T>::v8 x;
+  if (vec) {
+    x = *reinterpret_cast<const typename Elem<T>::v8*>(row + d0);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = row[(int64_t)(d0 + e) * sd];
+  }
+  return x;
+}
 
 template <typename T, int D>
 __global__ void __launch_bounds__(64) decode_partial_kernel(DecodeArgs a) {
   typedef typename Elem<T>::v8 v8;
-  constexpr int KK = D / 32;   // k-steps of the logits
-  constexpr int DT = D / 16;   // 16-column blocks of the output
-  constexpr int DPL = D / 64;  // elements of the new row per lane
-  constexpr int kRowBytes = D * (int)sizeof(T);
-  constexpr int kStepBytes = kDecStep * kRowBytes;
-  static_assert(kDecStep == 64, "four 16-key blocks per step");
+  constexpr int KK = D / 32;             // k-steps of the logits
+  constexpr int DT = D / 16;             // 16-column blocks of the output
+  constexpr int CPR = D / 8;             // 16-byte chunks per row
+  constexpr int GRP = 64 / CPR;          // rows per load round
+  constexpr int NVC = kDecTile / GRP;    // V chunks per lane and tile
+  constexpr int kVPitch = D + 16;        // as pass 1's V tile: transposing reads without bank conflicts
+  constexpr uint32_t kRowBytes = D * (uint32_t)sizeof(T);
   const int bh = blockIdx.x / a.S, split = blockIdx.x % a.S;
   const int b = bh / a.Hkv, hkv = bh % a.Hkv;
   const int g = a.Hq / a.Hkv;
   const int lane = threadIdx.x;
   const int li = lane & 15, lg = lane >> 4;
 
-  __shared__ __attribute__((aligned(16))) unsigned char ks_bytes[kStepBytes];
-  __shared__ __attribute__((aligned(16))) unsigned char vs_bytes[kStepBytes];
-  T* ks = reinterpret_cast<T*>(ks_bytes);
-  T* vs = reinterpret_cast<T*>(vs_bytes);
+  __shared__ __attribute__((aligned(16))) T vt[kDecTile * kVPitch];
 
   T* kb = static_cast<T*>(a.kbuf) + (int64_t)bh * a.C * D;
   T* vb = static_cast<T*>(a.vbuf) + (int64_t)bh * a.C * D;
-  const uint32_t head_bytes = (uint32_t)a.C * kRowBytes;
-  const rsrc_t krs = make_rsrc(kb, head_bytes), vrs = make_rsrc(vb, head_bytes);
-  // K and V rows j0 .. j0 + kDecStep - 1 to LDS (1 KB per instruction per wave).
-  auto issue_step = [&](int j0) __attribute__((always_inline)) {
-    const uint32_t src = (uint32_t)j0 * kRowBytes + 16u * lane;
-#pragma unroll 8
-    for (int it = 0; it < kStepBytes / 1024; ++it) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lds_void_t*)(ks_bytes + 1024 * it), 16, src + 1024u * it, 0, 0,
-                                               0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(vrs, (lds_void_t*)(vs_bytes + 1024 * it), 16, src + 1024u * it, 0, 0,
-                                               0);
-    }
-  };
+  const rsrc_t krs = make_rsrc(kb, (uint32_t)a.C * kRowBytes), vrs = make_rsrc(vb, (uint32_t)a.C * kRowBytes);
   const int k0 = split * a.kps;
-  issue_step(k0);
+  const uint32_t k_lane = li * kRowBytes + 16u * lg;
+  const int v_row = lane / CPR, v_col = 8 * (lane % CPR);
+  const uint32_t v_lane = v_row * kRowBytes + v_col * (uint32_t)sizeof(T);
+  v8 kop[2][KK];
+  u32x4 vch[NVC];
+  auto load_k = [&](int j0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk)
+        kop[h][kk] = bitcast_u4<v8>(buf_load16(krs, k_lane + (uint32_t)(j0 + 16 * h) * kRowBytes + 64u * kk));
+  };
+  auto load_v = [&](int j0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NVC; ++i) vch[i] = buf_load16(vrs, v_lane + (uint32_t)(j0 + i * GRP) * kRowBytes);
+  };
+  load_k(k0);
+  load_v(k0);
   const int n_in = *a.n_rows;
 
   // Q as the B operand: lane (li, lg) holds head li's elements 32 kk + 8 lg .. +7.
@@ -106,23 +128,21 @@ __global__ void __launch_bounds__(64) decode_partial_kernel(DecodeArgs a) {
     const bool hv = li < g;
     const T* qh = static_cast<const T*>(a.q) + (int64_t)b * a.q_sb + (int64_t)(hkv * g + (hv ? li : 0)) * a.q_sh;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk)
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        qop[kk][e] = hv ? qh[(int64_t)(32 * kk + 8 * lg + e) * a.q_sd] : static_cast<T>(0.f);
+    for (int kk = 0; kk < KK; ++kk) {
+      qop[kk] = load8(qh, 32 * kk + 8 * lg, a.q_sd, a.qvec);
+      if (!hv) qop[kk] = v8{};
+    }
   }
-  // The new row (element lane + 64 e).
+  // The new row, in the lanes' K operand and V chunk layouts.
   const T* kn = static_cast<const T*>(a.kn) + (int64_t)b * a.n_sb + (int64_t)hkv * a.n_sh;
   const T* vn = static_cast<const T*>(a.vn) + (int64_t)b * a.n_sb + (int64_t)hkv * a.n_sh;
-  T kn_r[DPL], vn_r[DPL];
+  v8 kx[KK];
 #pragma unroll
-  for (int e = 0; e < DPL; ++e) {
-    kn_r[e] = kn[(int64_t)(lane + 64 * e) * a.n_sd];
-    vn_r[e] = vn[(int64_t)(lane + 64 * e) * a.n_sd];
-  }
-
+  for (int kk = 0; kk < KK; ++kk) kx[kk] = load8(kn, 32 * kk + 8 * lg, a.n_sd, a.nvec);
+  const v8 vx = load8(vn, v_col, a.n_sd, a.nvec);
   const int n = min(n_in, a.C - 1);  // the host keeps n < C; the clamp keeps every access in bounds
   const int k1 = min(k0 + a.kps, n + 1);
+  const bool own_n = k0 <= n && n < k1;  // this split holds the new row
 
   float m = -INFINITY, lsum = 0.f;  // head li, log2 units; lsum is this lane's share
   f32x4 o[DT];
@@ -130,102 +150,91 @@ __global__ void __launch_bounds__(64) decode_partial_kernel(DecodeArgs a) {
   for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int tr_row = 4 * lg + li / 4, tr_col = 4 * (li % 4);
 
-  for (int j0 = k0; j0 < k1; j0 += kDecStep) {
-    if (j0 != k0) {
-      // The previous step's LDS reads must be done before the DMA writes land.
-      __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      issue_step(j0);
-    }
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const int nb = min(kDecStep, k1 - j0);
-    if (n >= j0 && n < j0 + kDecStep)  // row n (not stored yet) from the new row
+  for (int j0 = k0; j0 < k1; j0 += kDecTile) {
+    if (own_n && n < j0 + kDecTile) {
+      // The last tile, up to row n: the new row in its place, and V rows past
+      // it to zero (their p is 0, but 0 * NaN is not, and those rows hold
+      // whatever the buffer held).
 #pragma unroll
-      for (int e = 0; e < DPL; ++e) {
-        ks[(n - j0) * D + lane + 64 * e] = kn_r[e];
-        vs[(n - j0) * D + lane + 64 * e] = vn_r[e];
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk)
+          if (j0 + 16 * h + li == n) kop[h][kk] = kx[kk];
+#pragma unroll
+      for (int i = 0; i < NVC; ++i) {
+        const int row = j0 + v_row + i * GRP;
+        if (row == n) vch[i] = __builtin_bit_cast(u32x4, vx);
+        if (row > n) vch[i] = u32x4{0u, 0u, 0u, 0u};
       }
-    // V rows past the split's last key to zero: their p is 0, but 0 * NaN
-    // is not (the rows past n hold whatever the buffer held).
-    for (int c = nb * (kRowBytes / 16) + lane; c < kStepBytes / 16; c += 64)
-      reinterpret_cast<u32x4*>(vs_bytes)[c] = u32x4{0u, 0u, 0u, 0u};
-    __builtin_amdgcn_wave_barrier();
-
-    // S^T = K Q^T, 16 keys per block.
-    f32x4 s[4];
+    }
+    // S^T = K Q^T, 16 keys per block; then the K registers are free.
+    f32x4 s[2];
 #pragma unroll
-    for (int kb4 = 0; kb4 < 4; ++kb4) {
+    for (int h = 0; h < 2; ++h) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kk = 0; kk < KK; ++kk)
-        acc = Elem<T>::mfma(
-            bitcast_u4<v8>(*reinterpret_cast<const u32x4*>(ks + (16 * kb4 + li) * D + 32 * kk + 8 * lg)), qop[kk],
-            acc);
-      s[kb4] = acc;
+      for (int kk = 0; kk < KK; ++kk) acc = Elem<T>::mfma(kop[h][kk], qop[kk], acc);
+      s[h] = acc;
     }
-    // Keys past the split's last one masked; the head's step maximum over
+    load_k(j0 + kDecTile);
+#pragma unroll
+    for (int i = 0; i < NVC; ++i)
+      *reinterpret_cast<u32x4*>(vt + (v_row + i * GRP) * kVPitch + v_col) = vch[i];
+    load_v(j0 + kDecTile);
+    // Keys past the split's last one masked; the head's tile maximum over
     // its four lanes (IEEE maximum; scaling by a positive factor keeps the
     // order).
+    const int nb = k1 - j0;
     float tmax = -INFINITY;
 #pragma unroll
-    for (int kb4 = 0; kb4 < 4; ++kb4)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float x = (16 * kb4 + 4 * lg + r) < nb ? s[kb4][r] : -INFINITY;
-        s[kb4][r] = x;
+        const float x = (16 * h + 4 * lg + r) < nb ? s[h][r] : -INFINITY;
+        s[h][r] = x;
         tmax = __builtin_elementwise_maximum(tmax, x);
       }
     tmax = max_xor32(max_xor16(tmax)) * a.scale_log2;
     const float mnew = fmaxf(m, tmax);  // finite: key j0 is valid
     const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mnew);
-    float pv[16], psum = 0.f;
+    // P^T operand: element e is key 4 lg + e (e < 4) or 16 + 4 lg + e - 4; the
+    // transposing V reads below give V^T in that key order.
+    float psum = 0.f;
+    v8 phi, plo;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      pv[i] = __builtin_amdgcn_exp2f(fmaf(s[i / 4][i % 4], a.scale_log2, -mnew));
-      psum += pv[i];
+    for (int e = 0; e < 8; ++e) {
+      const float x = __builtin_amdgcn_exp2f(fmaf(s[e / 4][e % 4], a.scale_log2, -mnew));
+      psum += x;
+      phi[e] = static_cast<T>(x);
+      plo[e] = static_cast<T>(x - static_cast<float>(phi[e]));
     }
     lsum = lsum * alpha + psum;
     m = mnew;
+    if (wave_any(alpha != 1.f))
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
-    // P^T operands of the two 32-key k-steps: element e of k-step ks is key
-    // 32 ks + 4 lg + e (e < 4) or 32 ks + 16 + 4 lg + e - 4, which is
-    // pv[8 ks + e]; the transposing V reads below give V^T in that key order.
-    v8 phi[2], plo[2];
-#pragma unroll
-    for (int k2 = 0; k2 < 2; ++k2)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float x = pv[8 * k2 + e];
-        phi[k2][e] = static_cast<T>(x);
-        plo[k2][e] = static_cast<T>(x - static_cast<float>(phi[k2][e]));
-      }
+      for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
     // O^T += V^T P^T: lane (li, lg) of the A operand needs V[key][16 dt + li]
     // for the eight keys above; a transposing read gives output lane i of
     // each 16-lane group element e of input lane 4e + i/4's 8 bytes, element
     // i % 4, so input lane li reads key base + li/4, columns
     // 16 dt + 4 (li % 4) .. +3.
 #pragma unroll
-    for (int k2 = 0; k2 < 2; ++k2) {
+    for (int dt = 0; dt < DT; ++dt) {
       typedef short s4 __attribute__((ext_vector_type(4)));
       typedef __attribute__((address_space(3))) s4 lds_s4;
-      const T* vrow = vs + 32 * k2 * D;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const s4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(vrow + tr_row * D + 16 * dt + tr_col));
-        const s4 x1 =
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(vrow + (16 + tr_row) * D + 16 * dt + tr_col));
-        const v8 aop = __builtin_bit_cast(v8, __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
-        o[dt] = Elem<T>::mfma(aop, phi[k2], o[dt]);
-        o[dt] = Elem<T>::mfma(aop, plo[k2], o[dt]);
-      }
+      const s4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(vt + tr_row * kVPitch + 16 * dt + tr_col));
+      const s4 x1 =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(vt + (16 + tr_row) * kVPitch + 16 * dt + tr_col));
+      const v8 aop = __builtin_bit_cast(v8, __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
+      o[dt] = Elem<T>::mfma(aop, phi, o[dt]);
+      o[dt] = Elem<T>::mfma(aop, plo, o[dt]);
     }
   }
 
-  if (k0 <= n && n < k1)  // this split owns row n: store the new row
-#pragma unroll
-    for (int e = 0; e < DPL; ++e) {
-      kb[(int64_t)n * D + lane + 64 * e] = kn_r[e];
-      vb[(int64_t)n * D + lane + 64 * e] = vn_r[e];
+  if (own_n)  // store the new row
+    for (int d = lane; d < D; d += 64) {
+      kb[(int64_t)n * D + d] = kn[(int64_t)d * a.n_sd];
+      vb[(int64_t)n * D + d] = vn[(int64_t)d * a.n_sd];
     }
   // The split's partials (heads h < g).
   lsum = add_xor32(add_xor16(lsum));
@@ -233,9 +242,7 @@ __global__ void __launch_bounds__(64) decode_partial_kernel(DecodeArgs a) {
   if (li < g) {
     float* po = a.part_o + (base + li) * D + 4 * lg;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) po[16 * dt + r] = o[dt][r];
+    for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(po + 16 * dt) = o[dt];
     if (lg == 0) {
       a.part_m[base + li] = m;
       a.part_l[base + li] = lsum;
@@ -244,58 +251,76 @@ __global__ void __launch_bounds__(64) decode_partial_kernel(DecodeArgs a) {
 }
 
 // One wave per query head: combine the splits and write the output row.
-// Lane s holds split s's (m, l); the partial outputs of up to 32 splits are
-// loaded together with the statistics, before the reductions.
+// Lane s holds split s's (m, l); the partial outputs, 16 bytes a lane and so
+// two (D = 128) or four (D = 64) splits per load, are all issued together with
+// the statistics, before the reductions: one round trip whatever the number
+// of splits.  (One element a lane in batches of 32 splits took a second round
+// trip past 32: 12.8 against 11.5 us per layer, both kernels, at 57 splits of
+// 3300 rows, 32 query and 8 KV heads of 128.)
 template <typename T, int D>
 __global__ void __launch_bounds__(64) decode_merge_kernel(DecodeArgs a) {
-  constexpr int DPL = D / 64;
-  constexpr int kBatch = 32;
-  static_assert(kDecMaxSplits % kBatch == 0, "whole batches of splits");
+  constexpr int LPR = D / 4;                  // lanes per row
+  constexpr int SPL = 64 / LPR;               // splits per load
+  constexpr int NL = kDecMaxSplits / SPL;     // loads
   const int g = a.Hq / a.Hkv;
   const int b = blockIdx.x / a.Hq, hq = blockIdx.x % a.Hq;
   const int hkv = hq / g, h = hq % g;
   const int lane = threadIdx.x;
+  const int sub = lane / LPR, d0 = 4 * (lane % LPR);
   const int64_t base = ((int64_t)(b * a.Hkv + hkv) * a.S) * g + h;
-  float ob[kBatch][DPL];
-  auto load_batch = [&](int s0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u)
-#pragma unroll
-      for (int e = 0; e < DPL; ++e)
-        ob[u][e] = s0 + u < a.S ? a.part_o[(base + (int64_t)(s0 + u) * g) * D + lane * DPL + e] : 0.f;
-  };
   const float ml = lane < a.S ? a.part_m[base + (int64_t)lane * g] : -INFINITY;
   const float ll = lane < a.S ? a.part_l[base + (int64_t)lane * g] : 0.f;
-  load_batch(0);
+  // (Splits past the last read as zeros.)
+  const rsrc_t ors = make_rsrc(a.part_o + base * D, ((uint32_t)(a.S - 1) * g + 1) * D * 4u);
+  f32x4 ob[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i)
+    ob[i] = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(ors, ((uint32_t)(SPL * i + sub) * g * D + d0) * 4u, 0, 0));
   const float mx = wave_max_dpp(ml);
   // Lanes past S, and splits with no rows, weigh 0.
   const float f = ml == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml - mx);
   const float l = wave_sum_dpp(ll * f);
-  float acc[DPL];
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int e = 0; e < DPL; ++e) acc[e] = 0.f;
-  for (int s0 = 0; s0 < a.S; s0 += kBatch) {
-    if (s0) load_batch(s0);
+  for (int i = 0; i < NL; ++i)
+    if (i * SPL < a.S) {
+      const float fs = __shfl(f, SPL * i + sub);
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const float fs = read_lane_f(f, s0 + u);  // s0 + u < kDecMaxSplits <= 64
-#pragma unroll
-      for (int e = 0; e < DPL; ++e) acc[e] += fs * ob[u][e];
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(fs, ob[i][e], acc[e]);
     }
-  }
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  T* out = static_cast<T*>(a.out);
+  T* out = static_cast<T*>(a.out) + (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh;
 #pragma unroll
-  for (int e = 0; e < DPL; ++e) {
-    const int d = lane * DPL + e;
-    out[(int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)d * a.o_sd] = static_cast<T>(acc[e] * inv);
+  for (int e = 0; e < 4; ++e) {
+    float y = add_xor32(acc[e]);
+    if (SPL == 4) y = add_xor16(y);
+    if (sub == 0) out[(int64_t)(d0 + e) * a.o_sd] = static_cast<T>(y * inv);
   }
 }
 
-int decode_splits(int C) { return std::max(1, std::min(kDecMaxSplits, (C + kDecStep - 1) / kDecStep)); }
+// Splits of a cache of C rows for `heads` (b, kv head) pairs: whole tiles, and
+// no more waves than keep the memory busy, since each split also costs its
+// prologue, its epilogue and D floats per query head for the merge to read
+// (64 heads of 8004 rows, D = 128, both kernels: 50.1 us with 512 waves, 52.7
+// with 1024, 56.1 with 2048), two tiles a split at least (a short cache of 1639
+// rows, 2 heads, D = 64: 7.0 us a layer, against 8.7 with one tile a split and
+// 7.7 with four).
+constexpr int kDecWaves = 512;
+constexpr int kDecMinTiles = 2;
+
+struct DecodeSplits {
+  int S, kps;
+};
+static DecodeSplits decode_splits(int64_t heads, int C) {
+  const int tiles = (C + kDecTile - 1) / kDecTile;
+  const int want = (int)std::max<int64_t>(1, std::min<int64_t>(kDecMaxSplits, kDecWaves / heads));
+  const int per = std::max((tiles + want - 1) / want, std::min(tiles, kDecMinTiles));
+  return DecodeSplits{(tiles + per - 1) / per, per * kDecTile};
+}
 
 size_t decode_workspace_bytes(int B, int Hq, int Hkv, int D, int C) {
-  const size_t S = (size_t)decode_splits(C);
+  const size_t S = (size_t)decode_splits((int64_t)B * Hkv, C).S;
   const size_t rows = (size_t)B * Hkv * S * (Hq / Hkv);
   return rows * sizeof(float) * (2 + (size_t)D) + 256;
 }
@@ -329,14 +354,20 @@ hipError_t launch_decode_attention(const DecodeParams& p, hipStream_t st) {
   a.Hkv = p.Hkv;
   a.D = p.D;
   a.C = p.C;
-  a.S = decode_splits(p.C);
-  a.kps = (p.C + a.S - 1) / a.S;
+  const DecodeSplits sp = decode_splits((int64_t)p.B * p.Hkv, p.C);
+  a.S = sp.S;
+  a.kps = sp.kps;
   a.scale_log2 = p.scale * 1.4426950408889634f;
   const size_t rows = (size_t)p.B * p.Hkv * a.S * (p.Hq / p.Hkv);
-  char* ws = static_cast<char*>(p.workspace);
+  char* ws = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(p.workspace) + 15) & ~(uintptr_t)15);
+  auto vec = [](const void* x, int64_t sb, int64_t sh, int64_t sd) {
+    return (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && sd == 1 && sb % 8 == 0 && sh % 8 == 0;
+  };
+  a.qvec = vec(p.q, p.q_sb, p.q_sh, p.q_sd);
+  a.nvec = vec(p.kn, p.n_sb, p.n_sh, p.n_sd) && vec(p.vn, p.n_sb, p.n_sh, p.n_sd);
   a.part_m = reinterpret_cast<float*>(ws);
   a.part_l = a.part_m + rows;
-  a.part_o = a.part_l + rows;
+  a.part_o = a.part_m + ((2 * rows + 3) & ~(size_t)3);  // 16-byte stores
   a.out = p.out;
   a.o_sb = p.o_sb;
   a.o_sh = p.o_sh;

@@ -127,7 +127,6 @@ struct DecodeParams {
   int64_t o_sb, o_sh, o_sd;
   void* workspace;
 };
-int decode_splits(int C);
 size_t decode_workspace_bytes(int B, int Hq, int Hkv, int D, int C);
 hipError_t launch_decode_attention(const DecodeParams& p, hipStream_t st);
 

@@ -183,3 +183,31 @@ def test_decoder_graph_replays_equal_eager_steps(gpu, tiny):
         tok = a[:, -1].argmax(-1, keepdim=True)
     with pytest.raises(RuntimeError, match="capacity"):
         graph.step(tok)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,C,n,aligned", [
+    (1, 4, 2, 64, 33, 32, True),       # the new row alone in the second tile
+    (1, 4, 2, 128, 64, 31, False),     # the new row ends the first tile; scalar loads of q and the new row
+    (1, 2, 1, 128, 4096, 4095, True),  # 64 splits of two tiles, buffer full
+    (40, 16, 16, 64, 96, 70, True),    # 640 heads: one split each, the third tile partial
+    (3, 14, 2, 64, 2000, 1984, False),  # 32 splits of two tiles, the last ones empty
+])
+def test_tiles_and_splits(gpu, B, Hq, Hkv, D, C, n, aligned):
+    """Edges of the 32-key tiles and of the splits (at least two tiles each),
+    NaN in every row from the new one's position on, and rows that do not
+    allow 16-byte loads."""
+    from dropkv_amd import ops
+    g = torch.Generator().manual_seed(C)
+    kb, vb = (torch.randn(B, Hkv, C, D, generator=g).bfloat16().to(gpu) for _ in range(2))
+    kb[:, :, n:] = float("nan")
+    vb[:, :, n:] = float("nan")
+    pad = 0 if aligned else 1
+    q, kn, vn = (torch.randn(B, h, 1, D + pad, generator=g).bfloat16().to(gpu)[..., pad:] for h in (Hq, Hkv, Hkv))
+    k_rows, v_rows = (torch.cat([x[:, :, :n].clone(), y], dim=2) for x, y in ((kb, kn), (vb, vn)))
+    out = torch.empty(B, 1, Hq, D, dtype=torch.bfloat16, device=gpu)
+    ops.decode_attention(q, kn, vn, kb, vb, torch.tensor([n], dtype=torch.int32, device=gpu), D ** -0.5, out,
+                         ops.decode_workspace(B, Hq, Hkv, D, C, gpu))
+    ref = _ref_attention(q, k_rows, v_rows, D ** -0.5)
+    # bf16 output: half an ulp (2^-9) of it, and the same of the weights' sum
+    torch.testing.assert_close(out.float(), ref, rtol=2 ** -7, atol=2 ** -9)
+    assert torch.equal(kb[:, :, n], kn[:, :, 0]) and torch.equal(vb[:, :, n], vn[:, :, 0])
