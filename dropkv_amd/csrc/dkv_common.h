@@ -100,6 +100,28 @@ __device__ __forceinline__ i32x2 buf_load8i(rsrc_t r, uint32_t voff) {
   return __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0));
 }
 
+// Division of n < 2^31 by a divisor d known to the host: n / d = (n m) >> (31 + s)
+// with s = ceil(log2 d), m = ceil(2^(31+s) / d) < 2^32 (m d exceeds 2^(31+s) by
+// less than d <= 2^s, which moves the quotient by less than n 2^s / 2^(31+s) < 1
+// over d).  Two multiplies and a shift, where the compiler's integer division
+// by a kernel argument is a chain of ~25 dependent operations through a float
+// reciprocal.
+struct Div {
+  uint32_t m, s, d;
+  __host__ __device__ static Div of(uint32_t d) {
+    uint32_t s = 0;
+    while ((uint64_t(1) << s) < d) ++s;
+    return Div{(uint32_t)(((uint64_t(1) << (31 + s)) + d - 1) / d), s, d};
+  }
+  __host__ __device__ int div(int n) const { return (int)(((uint64_t)(uint32_t)n * m) >> (31 + s)); }
+  __host__ __device__ int mod(int n) const { return n - div(n) * (int)d; }
+};
+
+// The divisors of a scoring kernel's grid and rows.
+struct ScoreDiv {
+  Div n_mc, splits, hkv, w;
+};
+
 // Where the rows of K and of V lie: row r of (batch b, KV head h) starts at
 // element b * sb + h * sh of the tensor plus r * rb bytes.  The kernels take
 // any such layout (a head's rows one after the other, or the [B, L, H, D]

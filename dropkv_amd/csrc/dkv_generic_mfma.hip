@@ -31,7 +31,10 @@
 // different rows) and gave each query row a workgroup of its own: 3990 us for
 // 8192 keys of D 256 in bf16 (8 query, 4 KV heads), 3650 us for 8192 keys of D
 // 64 in fp32 (14, 2), 1790 us for 4099 keys of D 96 in fp16 (16, 16); these
-// kernels take 49, 34 and 34 us.
+// kernels take 37, 29 and 32 us.  With the operand loads issued one round trip
+// after the other (a wait for a load waits for every earlier one, so the query
+// rows go before K and V), Q and Y staged 32 rows at a time and y's columns 64
+// words apart in LDS they took 49, 34 and 34 us.
 //
 // Kernels (fp32 inputs, or no p rounding: 1, 3, 4; else 1, 2, 3, 4):
 //   1. part<kFlash>: per (head, 32 query rows, key split) the row maxima, sums
@@ -57,6 +60,9 @@ constexpr float kDirect = 0.25f;  // dist2 below this share of its terms is take
 
 // Chunks whose loads a wave issues together (those past D are no request).
 constexpr int kGrp = 8;
+
+// Groups of waves that share a step's keys when CG of them share the columns.
+__host__ __device__ constexpr int part_kg(int CG) { return CG == 1 ? 8 : CG == 2 ? 4 : 2; }
 
 enum { kStats = 0, kSum = 1, kFlash = 2 };
 
@@ -114,27 +120,23 @@ __device__ __forceinline__ f32x4 load4(rsrc_t r, uint32_t off) {
 
 constexpr uint32_t kPastAll = 0xfffffff0u;  // an offset past every view: zeros, no memory request
 
-// Query rows m0 .. m0 + 16 * kRB - 1 as MFMA operands in LDS: slot (rb, chunk,
-// lane) holds the lane's 16 bytes; zeros past row M and column D.
-template <typename T, int kRB, int NT>
-__device__ __forceinline__ void stage_q(u32x4* qop, int nch, const T* __restrict__ q, int64_t q_sb, int64_t q_sh,
-                                        int64_t q_ss, int64_t q_sd, int b, int hkv, int g, int W, int Lq, int M,
-                                        int D, int m0) {
-  for (int s = threadIdx.x; s < kRB * nch * 64; s += NT) {
-    const int lane = s & 63, c = (s >> 6) % nch, rb = (s >> 6) / nch;
-    const int m = m0 + 16 * rb + (lane & 15), d0 = c * kCols<T> + kEpl<T> * (lane >> 4);
-    T x[kEpl<T>];
-    const int mm = min(m, M - 1);
-    const T* row = q + (int64_t)b * q_sb + (int64_t)(hkv * g + mm / W) * q_sh + (int64_t)(Lq - W + mm % W) * q_ss;
+// Where query row m of the group starts (rows past M: the last one).
+template <typename T>
+__device__ __forceinline__ const T* q_row(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int b,
+                                          int hkv, int g, const Div& dw, int Lq, int M, int m) {
+  const int mm = min(m, M - 1), gi = dw.div(mm);
+  return q + (int64_t)b * q_sb + (int64_t)(hkv * g + gi) * q_sh + (int64_t)(Lq - (int)dw.d + mm - gi * (int)dw.d) * q_ss;
+}
+
+// A lane's 16 bytes of an MFMA operand: kEpl elements of a row by stride.
+template <typename T>
+__device__ __forceinline__ u32x4 gather_unit(const T* row, int64_t sd) {
+  T x[kEpl<T>];
 #pragma unroll
-    for (int e = 0; e < kEpl<T>; ++e) x[e] = row[(int64_t)min(d0 + e, D - 1) * q_sd];
-#pragma unroll
-    for (int e = 0; e < kEpl<T>; ++e)
-      if (m >= M || d0 + e >= D) x[e] = static_cast<T>(0.f);
-    u32x4 w;
-    __builtin_memcpy(&w, x, 16);
-    qop[s] = w;
-  }
+  for (int e = 0; e < kEpl<T>; ++e) x[e] = row[(int64_t)e * sd];
+  u32x4 w;
+  __builtin_memcpy(&w, x, 16);
+  return w;
 }
 
 }  // namespace
@@ -151,11 +153,11 @@ __device__ __forceinline__ void stage_q(u32x4* qop, int nch, const T* __restrict
 // ---------------------------------------------------------------------------
 template <typename T, int kRB, int kMode>
 __global__ void __launch_bounds__(64 * kPartWaves)
-genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd,
+genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd, bool qvec,
                  const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs, int Hkv, int Lq, int Lk, int D,
                  int W, int g, int M, int n_mc, int n_splits, int kps, float scale_log2,
-                 float* __restrict__ part_ml, float* __restrict__ part_y, float* __restrict__ row_mr) {
-  constexpr int NT = 64 * kPartWaves;
+                 float* __restrict__ part_ml, float* __restrict__ part_y, float* __restrict__ row_mr,
+                 ScoreDiv dv) {
   constexpr int R = 16 * kRB;
   extern __shared__ u32x4 gm_lds[];
   __shared__ float wred[2][kPartWaves][kRowsC];
@@ -165,8 +167,9 @@ genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
   float* P = reinterpret_cast<float*>(qop + kRB * nch * 64);
 
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int mc = lid % n_mc, split = (lid / n_mc) % n_splits, head = lid / (n_mc * n_splits);
-  const int b = head / Hkv, hkv = head % Hkv;
+  const int mc = dv.n_mc.mod(lid), hs = dv.n_mc.div(lid);
+  const int split = dv.splits.mod(hs), head = dv.splits.div(hs);
+  const int b = dv.hkv.div(head), hkv = dv.hkv.mod(head);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, li = lane & 15, lg = lane >> 4;
   const int k_begin = split * kps, k_end = min(k_begin + kps, Lk), nrel = k_end - k_begin;
   const rsrc_t krs = make_rsrc(reinterpret_cast<const char*>(kp + b * kvs.k_sb + hkv * kvs.k_sh) +
@@ -177,20 +180,86 @@ genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
                                rows_bytes(nrel, kvs.v_rb, D * (uint32_t)sizeof(T)));
   const int64_t slot = ((int64_t)head * n_mc + mc) * n_splits + split;
 
-  stage_q<T, kRB, NT>(qop, nch, q, q_sb, q_sh, q_ss, q_sd, b, hkv, g, W, Lq, M, D, mc * kRowsC);
+  // Loads of the wave's 32 keys at t, chunks c0 .. c0 + kGrp - 1, and of 32 keys
+  // of its share of V from row t of a step; the first of both are on their way
+  // while the operands are staged.
+  u32x4 k0[kGrp], k1[kGrp];
+  auto load_k = [&](int t, int c0) __attribute__((always_inline)) {
+    const uint32_t r0 = (uint32_t)(t + li) * kvs.k_rb, r1 = r0 + 16u * kvs.k_rb;
+#pragma unroll
+    for (int u = 0; u < kGrp; ++u) {
+      const int col = (c0 + u) * kCols<T> + kEpl<T> * lg;
+      const uint32_t cb = col * (uint32_t)sizeof(T);
+      k0[u] = buf_load16(krs, col < D ? r0 + cb : kPastAll);
+      k1[u] = buf_load16(krs, col < D ? r1 + cb : kPastAll);
+    }
+  };
+  const int CG = (D + 63) / 64, KG = part_kg(CG), kpg = kPartKeys / kPartWaves * (CG == 3 ? 4 : CG);
+  const int kg = CG == 3 ? (wv * 11) >> 5 : wv >> (CG / 2), cg = wv - kg * CG;  // wv / CG, wv % CG
+  const uint32_t v_col = 64 * cg + 4 * li;
+  auto load_v = [&](f32x4 (&v)[2][4], int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[h][e] = load4<T>(vrs, v_col < (uint32_t)D && kg < KG
+                                    ? (uint32_t)(t + 16 * h + 4 * lg + e) * kvs.v_rb + v_col * (uint32_t)sizeof(T)
+                                    : kPastAll);
+  };
+  f32x4 va[2][4], vb[2][4];
+  // A wait for a load also waits for every load issued before it: the query
+  // rows (and the splits' statistics) first, then K and V.  Slot (rb, chunk,
+  // lane) of qop holds the lane's 16 bytes; wave w takes chunks w and w + 8.
+  static_assert(2 * kPartWaves * kCols<float> >= 256, "two chunks a wave");
+  u32x4 qr[kRB][2];
+  const T* qrow[kRB];
+#pragma unroll
+  for (int rb = 0; rb < kRB; ++rb)
+    qrow[rb] = q_row(q, q_sb, q_sh, q_ss, b, hkv, g, dv.w, Lq, M, mc * kRowsC + 16 * rb + li);
+  const int qd = wv * kCols<T> + kEpl<T> * lg;  // column of the wave's first chunk
+  if (qvec)
+#pragma unroll
+    for (int rb = 0; rb < kRB; ++rb)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int d0 = qd + i * kPartWaves * kCols<T>;
+        qr[rb][i] = *reinterpret_cast<const u32x4*>(qrow[rb] + (d0 < D ? d0 : 0));
+      }
+  constexpr int kMl = 4;  // splits per thread read up front (16 threads a row)
+  f32x2 mlv[kMl];
+  const rsrc_t mrs = make_rsrc(part_ml + ((int64_t)head * n_mc + mc) * n_splits * kRowsC * 2,
+                               (uint32_t)n_splits * kRowsC * 8u);
+  const int srow = tid >> 4;  // the row whose statistics this thread helps to combine
+  if constexpr (kMode == kSum)
+#pragma unroll
+    for (int i = 0; i < kMl; ++i) mlv[i] = buf_load8f(mrs, ((uint32_t)((tid & 15) + 16 * i) * kRowsC + srow) * 8u);
+  load_k(32 * wv, 0);
+  if constexpr (kMode != kStats) load_v(va, kg * kpg);
+#pragma unroll
+  for (int rb = 0; rb < kRB; ++rb)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (wv + kPartWaves * i < nch) {
+        const int d0 = qd + i * kPartWaves * kCols<T>;
+        if (!qvec) qr[rb][i] = gather_unit(qrow[rb] + (int64_t)(d0 < D ? d0 : 0) * q_sd, q_sd);
+        qop[(rb * nch + wv + kPartWaves * i) * 64 + lane] =
+            mc * kRowsC + 16 * rb + li < M && d0 < D ? qr[rb][i] : u32x4{0u, 0u, 0u, 0u};
+      }
   if constexpr (kMode == kSum) {
-    // The rows' log-sum-exp from the splits' maxima and sums: 16 threads a row.
-    const int row = tid >> 4;
-    const float* ml = part_ml + (((int64_t)head * n_mc + mc) * n_splits) * kRowsC * 2;
+    // The rows' maxima and sums from the splits': 16 threads a row.
+    const int row = srow, s0 = tid & 15;
     float mx = -INFINITY;
-    for (int s = tid & 15; s < n_splits; s += 16) mx = fmaxf(mx, ml[(s * kRowsC + row) * 2]);
+#pragma unroll
+    for (int i = 0; i < kMl; ++i) mx = s0 + 16 * i < n_splits ? fmaxf(mx, mlv[i][0]) : mx;
+    for (int s = s0 + 16 * kMl; s < n_splits; s += 16)
+      mx = fmaxf(mx, buf_load8f(mrs, ((uint32_t)s * kRowsC + row) * 8u)[0]);
 #pragma unroll
     for (int o = 8; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
     float l = 0.f;
-    for (int s = tid & 15; s < n_splits; s += 16) {
-      const float m = ml[(s * kRowsC + row) * 2];
-      if (m != -INFINITY) l += ml[(s * kRowsC + row) * 2 + 1] * exp2f((m - mx) * scale_log2);
-    }
+    auto part = [&](f32x2 p) { return p[0] == -INFINITY ? 0.f : p[1] * exp2f((p[0] - mx) * scale_log2); };
+#pragma unroll
+    for (int i = 0; i < kMl; ++i) l += s0 + 16 * i < n_splits ? part(mlv[i]) : 0.f;
+    for (int s = s0 + 16 * kMl; s < n_splits; s += 16) l += part(buf_load8f(mrs, ((uint32_t)s * kRowsC + row) * 8u));
 #pragma unroll
     for (int o = 8; o >= 1; o >>= 1) l += __shfl_xor(l, o);
     if ((tid & 15) == 0) {
@@ -206,7 +275,7 @@ genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
 #pragma unroll
   for (int rb = 0; rb < kRB; ++rb) {
     const int m = mc * kRowsC + 16 * rb + li;
-    bound[rb] = m < M ? Lk - W + m % W : -1;
+    bound[rb] = m < M ? Lk - W + dv.w.mod(m) : -1;
   }
   // Row 16 rb + li: the maximum (so far), and this lane's share of the sum
   // (kSum: the reciprocal of the row's sum).
@@ -217,8 +286,6 @@ genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
     lsum[rb] = kMode == kSum ? row_r[16 * rb + li] : 0.f;
   }
   // The waves' shares of Y^T: columns 64 cg .. +63, keys kg * kpg .. of a step.
-  const int CG = (D + 63) / 64, KG = kPartWaves / CG, kpg = kPartKeys / KG;
-  const int cg = wv % CG, kg = wv / CG;
   f32x4 yacc[4][kRB];
 #pragma unroll
   for (int c = 0; c < 4; ++c)
@@ -232,28 +299,19 @@ genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int rb = 0; rb < kRB; ++rb) s[kb][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (tw < nrel) {
-      const uint32_t r0 = (uint32_t)(tw + li) * kvs.k_rb, r1 = r0 + 16u * kvs.k_rb;
-      for (int c0 = 0; c0 < nch; c0 += kGrp) {
-        u32x4 k0[kGrp], k1[kGrp];
+    for (int c0 = 0; c0 < nch; c0 += kGrp) {
+      if (c0) load_k(tw, c0);
 #pragma unroll
-        for (int u = 0; u < kGrp; ++u) {
-          const int col = (c0 + u) * kCols<T> + kEpl<T> * lg;
-          const uint32_t cb = col * (uint32_t)sizeof(T);
-          k0[u] = buf_load16(krs, col < D ? r0 + cb : kPastAll);
-          k1[u] = buf_load16(krs, col < D ? r1 + cb : kPastAll);
-        }
+      for (int u = 0; u < kGrp; ++u)
+        if (c0 + u < nch)
 #pragma unroll
-        for (int u = 0; u < kGrp; ++u)
-          if (c0 + u < nch)
-#pragma unroll
-            for (int rb = 0; rb < kRB; ++rb) {
-              const u32x4 qf = qop[(rb * nch + c0 + u) * 64 + lane];
-              s[0][rb] = mfma_chunk<T>(k0[u], qf, s[0][rb]);
-              s[1][rb] = mfma_chunk<T>(k1[u], qf, s[1][rb]);
-            }
-      }
+          for (int rb = 0; rb < kRB; ++rb) {
+            const u32x4 qf = qop[(rb * nch + c0 + u) * 64 + lane];
+            s[0][rb] = mfma_chunk<T>(k0[u], qf, s[0][rb]);
+            s[1][rb] = mfma_chunk<T>(k1[u], qf, s[1][rb]);
+          }
     }
+    if (t0 + kPartKeys < nrel) load_k(tw + kPartKeys, 0);
     float tm[kRB];
 #pragma unroll
     for (int rb = 0; rb < kRB; ++rb) {
@@ -320,18 +378,10 @@ genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
       }
       __syncthreads();
       if (kg < KG) {
-        const uint32_t col = 64 * cg + 4 * li;
-        const uint32_t cb = col * (uint32_t)sizeof(T);
+        // 32 keys at a time, the next 32 on their way (the last ones of a step:
+        // the next step's first).
         const int n = min(kpg, nrel - t0 - kg * kpg);
-        for (int kk = 0; kk < n; kk += 32) {
-          f32x4 v[2][4];
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              v[h][e] = load4<T>(vrs, col < (uint32_t)D
-                                          ? (uint32_t)(t0 + kg * kpg + kk + 16 * h + 4 * lg + e) * kvs.v_rb + cb
-                                          : kPastAll);
+        auto add = [&](const f32x4 (&v)[2][4], int kk) __attribute__((always_inline)) {
 #pragma unroll
           for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -343,6 +393,21 @@ genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
 #pragma unroll
                 for (int c = 0; c < 4; ++c) yacc[c][rb] = mfma_f32(v[h][e][c], p[e], yacc[c][rb]);
             }
+        };
+        const int next = t0 + kPartKeys + kg * kpg;
+        for (int kk = 0; kk < kpg; kk += 64) {
+          const int r = t0 + kg * kpg + kk;
+          load_v(vb, kk + 32 < kpg ? r + 32 : next);
+          if (kk < n) add(va, kk);
+          if (kk + 32 < kpg) {
+            load_v(va, kk + 64 < kpg ? r + 64 : next);
+            if (kk + 32 < n) add(vb, kk + 32);
+          } else {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) va[h][e] = vb[h][e];
+          }
         }
       }
       __syncthreads();  // P and wred are rewritten by the next step
@@ -373,7 +438,7 @@ genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
     // Y of the KG key groups, added in order (over the operands and P, dead
     // since the last step's barrier).
     float* yb = reinterpret_cast<float*>(gm_lds);
-    const int pitch = 64 * CG;
+    const int pitch = 64 * CG + 4;  // (rows of 64 words would share their banks)
     if (kg < KG)
 #pragma unroll
       for (int rb = 0; rb < kRB; ++rb)
@@ -382,9 +447,8 @@ genm_part_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_
           *reinterpret_cast<f32x4*>(yb + (kg * R + 16 * rb + li) * pitch + 64 * cg + 16 * lg + 4 * r) =
               f32x4{yacc[0][rb][r], yacc[1][rb][r], yacc[2][rb][r], yacc[3][rb][r]};
     __syncthreads();
-    const int d4 = D / 4;
-    for (int i = tid; i < R * d4; i += NT) {
-      const int row = i / d4, d = 4 * (i % d4);
+    const int d = 4 * lane;
+    for (int row = wv; row < R && d < D; row += kPartWaves) {
       f32x4 y = *reinterpret_cast<const f32x4*>(yb + row * pitch + d);
       for (int k = 1; k < KG; ++k) y += *reinterpret_cast<const f32x4*>(yb + (k * R + row) * pitch + d);
       *reinterpret_cast<f32x4*>(part_y + (slot * kRowsC + row) * D + d) = y;
@@ -401,12 +465,11 @@ __global__ void __launch_bounds__(64)
 genm_merge_kernel(const float* __restrict__ part_ml, const float* __restrict__ part_y, int n_mc, int n_splits, int M,
                   int D, float scale_log2, int flash, int y_round, float* __restrict__ ystat, float* __restrict__ yf32,
                   float* __restrict__ row_mr, uint32_t* __restrict__ zero_ptr, int64_t zero_words) {
-  const int lane = threadIdx.x, head = blockIdx.x / M, m = blockIdx.x % M;
+  const int lane = threadIdx.x, head = blockIdx.y, m = blockIdx.x;
   const int mc = m / kRowsC, row = m % kRowsC;
   const int64_t slot0 = ((int64_t)head * n_mc + mc) * n_splits;
   const float* ml = part_ml + (slot0 * kRowsC + row) * 2;
   const bool col = 4 * lane < D;
-  const float* py = part_y + (slot0 * kRowsC + row) * D + (col ? 4 * lane : 0);
   float mx = -INFINITY;
   for (int s = lane; s < n_splits; s += 64) mx = fmaxf(mx, ml[s * kRowsC * 2]);
   mx = wave_max_dpp(mx);
@@ -416,14 +479,26 @@ genm_merge_kernel(const float* __restrict__ part_ml, const float* __restrict__ p
     if (ms != -INFINITY) l += ml[s * kRowsC * 2 + 1] * exp2f((ms - mx) * scale_log2);
   }
   l = wave_sum_dpp(l);
+  // y in batches of 32 splits whose loads are all issued together (zeros past
+  // the last split and past column D).
+  const rsrc_t yrs = make_rsrc(part_y + slot0 * kRowsC * D, (uint32_t)n_splits * kRowsC * D * 4u);
   f32x4 y = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-  for (int s = 0; s < n_splits; ++s) {
-    const f32x4 ys = *reinterpret_cast<const f32x4*>(py + (int64_t)s * kRowsC * D);
-    const float ms = ml[s * kRowsC * 2];
-    const float f = !flash ? 1.f : ms == -INFINITY ? 0.f : exp2f((ms - mx) * scale_log2);
+  for (int s0 = 0; s0 < n_splits; s0 += 32) {
+    f32x4 ys[32];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] = fmaf(f, ys[e], y[e]);
+    for (int u = 0; u < 32; ++u)
+      ys[u] = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     yrs, 4 * lane < D && s0 + u < n_splits ? (((uint32_t)(s0 + u) * kRowsC + row) * D + 4 * lane) * 4u
+                                                            : kPastAll, 0, 0));
+    const float ms = s0 + (lane & 31) < n_splits ? ml[(s0 + (lane & 31)) * kRowsC * 2] : -INFINITY;
+    const float fl = !flash ? 1.f : ms == -INFINITY ? 0.f : exp2f((ms - mx) * scale_log2);
+#pragma unroll
+    for (int u = 0; u < 32; ++u) {
+      const float f = read_lane_f(fl, u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = fmaf(f, ys[u][e], y[e]);
+    }
   }
   const int mpad = n_mc * kRowsC;
   const int64_t rbase = (int64_t)head * mpad + m;
@@ -443,174 +518,201 @@ genm_merge_kernel(const float* __restrict__ part_ml, const float* __restrict__ p
     if (flash) reinterpret_cast<float2*>(row_mr)[rbase] = make_float2(mx, rl);  // (else part<kSum> wrote them)
   }
   if (zero_ptr)
-    for (int64_t i = (int64_t)blockIdx.x * 64 + lane; i < zero_words; i += (int64_t)gridDim.x * 64) zero_ptr[i] = 0u;
+    for (int64_t i = ((int64_t)head * M + m) * 64 + lane; i < zero_words; i += (int64_t)gridDim.x * gridDim.y * 64)
+      zero_ptr[i] = 0u;
 }
 
 // ---------------------------------------------------------------------------
 // Scores.  One workgroup per (head, kpw keys); a wave takes 16 keys at a time:
 // S = Q K^T and G = Y V^T with rows on the result registers and keys on the
 // lanes, so that a key's sum over the rows is in-lane but for the four lane
-// groups.  Q and Y of 16 * kRB rows at a time in LDS in operand order; the
-// keys' sums over earlier rows in LDS.  kYT: Y was rounded to T, so T operands
-// hold it exactly.
+// groups.  Q and Y of `rs` rows at a time (all of them where LDS allows) in
+// operand order; a tile's K and V stay in registers for all of them (up to
+// eight chunks); the keys' sums over earlier rows in LDS.  kYT: Y was rounded
+// to T, so T operands hold it exactly.
 // ---------------------------------------------------------------------------
 template <typename T, int kRB, bool kYT>
 __global__ void __launch_bounds__(64 * kScoreWaves)
-genm_score_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd,
+genm_score_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd, bool qvec,
                   const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs, int Hkv, int Lq, int Lk, int D,
-                  int W, int g, int M, int mpad, float scale_log2, float eps, int p_round, int wgs, int kpw,
+                  int W, int g, int M, int mpad, float scale_log2, float eps, int p_round, int kpw, int rs,
                   const float* __restrict__ ystat, const float* __restrict__ yf32, const float* __restrict__ row_mr,
-                  float* __restrict__ scores) {
+                  float* __restrict__ scores, ScoreDiv dv) {
   constexpr int NT = 64 * kScoreWaves;
   constexpr int R = 16 * kRB;
   constexpr int YV = kYT ? 1 : kEpl<T> / 4;  // 16-byte units of Y per lane and chunk
   extern __shared__ u32x4 gm_lds[];
-  __shared__ __attribute__((aligned(16))) float row_m[kRowsC], row_r[kRowsC];
-  __shared__ __attribute__((aligned(16))) float yn2[kRowsC];
   const int nch = (D + kCols<T> - 1) / kCols<T>;
-  u32x4* qop = gm_lds;
-  u32x4* yop = qop + kRB * nch * 64;                          // [kRB][nch][YV][64]
-  float* sc = reinterpret_cast<float*>(yop + kRB * nch * YV * 64);  // [kpw]
+  u32x4* qop = gm_lds;                                        // [rs / 16][nch][64]
+  u32x4* yop = qop + rs / 16 * nch * 64;                      // [rs / 16][nch][YV][64]
+  f32x4* st = reinterpret_cast<f32x4*>(yop + rs / 16 * nch * YV * 64);  // [rs / 16][3][4]: maxima, 1 / sums, |y|^2
+  float* stf = reinterpret_cast<float*>(st);
+  float* sc = stf + rs * 3;                                   // [kpw]
 
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int head = lid / wgs, k_begin = (lid % wgs) * kpw, nrel = min(kpw, Lk - k_begin);
-  const int b = head / Hkv, hkv = head % Hkv;
+  const int head = dv.splits.div(lid), k_begin = dv.splits.mod(lid) * kpw, nrel = min(kpw, Lk - k_begin);
+  const int b = dv.hkv.div(head), hkv = dv.hkv.mod(head);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, li = lane & 15, lg = lane >> 4;
   const rsrc_t krs = make_rsrc(reinterpret_cast<const char*>(kp + b * kvs.k_sb + hkv * kvs.k_sh) +
                                    (int64_t)k_begin * kvs.k_rb,
                                rows_bytes(nrel, kvs.k_rb, D * (uint32_t)sizeof(T)));
   const char* vhead = reinterpret_cast<const char*>(vp + b * kvs.v_sb + hkv * kvs.v_sh) + (int64_t)k_begin * kvs.v_rb;
   const rsrc_t vrs = make_rsrc(vhead, rows_bytes(nrel, kvs.v_rb, D * (uint32_t)sizeof(T)));
-  const float inv_g = static_cast<float>(g);
 
-  for (int r0 = 0; r0 < M; r0 += R) {
+  u32x4 kf[kGrp], vf[kGrp];
+  auto load = [&](int t, int c0) __attribute__((always_inline)) {
+    const uint32_t kr = (uint32_t)(t + li) * kvs.k_rb, vr = (uint32_t)(t + li) * kvs.v_rb;
+#pragma unroll
+    for (int u = 0; u < kGrp; ++u) {
+      const int col = (c0 + u) * kCols<T> + kEpl<T> * lg;
+      const uint32_t cb = col * (uint32_t)sizeof(T);
+      kf[u] = buf_load16(krs, col < D ? kr + cb : kPastAll);
+      vf[u] = buf_load16(vrs, col < D ? vr + cb : kPastAll);
+    }
+  };
+  const bool once = nch <= kGrp;  // a tile's K and V fit the registers
+
+  for (int r0 = 0; r0 < M; r0 += rs) {
     if (r0) __syncthreads();  // the previous rows' operands are dead
-    stage_q<T, kRB, NT>(qop, nch, q, q_sb, q_sh, q_ss, q_sd, b, hkv, g, W, Lq, M, D, r0);
+    const int nrb = min(rs, (M - r0 + R - 1) / R * R) / 16;
     const float* yrow0 = yf32 + ((int64_t)head * mpad + r0) * D;
-    for (int s = tid; s < kRB * nch * 64; s += NT) {
-      const int l = s & 63, c = (s >> 6) % nch, rb = (s >> 6) / nch;
-      const int row = 16 * rb + (l & 15), d0 = c * kCols<T> + kEpl<T> * (l >> 4);
-      const bool in = r0 + row < M && d0 < D;  // (D is a multiple of kEpl)
-      float y[kEpl<T>];
+    // Q and Y, kRB row blocks and eight chunks at a time (wave w takes chunks w
+    // and w + 4), every load of a batch issued before its first LDS write, and
+    // the first tile's K and V behind the first batch's.
+    constexpr int YU = kEpl<T> / 4;
+    for (int rb0 = 0; rb0 < nrb; rb0 += kRB)
+      for (int c0 = 0; c0 < nch; c0 += 2 * kScoreWaves) {
+        u32x4 qr[kRB][2];
+        f32x4 yr[kRB][2][YU];
+        const T* qrow[kRB];
+        const int qd = (c0 + wv) * kCols<T> + kEpl<T> * lg;
 #pragma unroll
-      for (int e = 0; e < kEpl<T>; ++e) y[e] = in ? yrow0[(int64_t)row * D + d0 + e] : 0.f;
-      if constexpr (kYT) {
-        T x[kEpl<T>];
+        for (int i = 0; i < kRB; ++i) {
+          const int m = r0 + 16 * (rb0 + i) + li;
+          qrow[i] = q_row(q, q_sb, q_sh, q_ss, b, hkv, g, dv.w, Lq, M, m);
+          const float* yrow = yrow0 + (int64_t)(min(m, M - 1) - r0) * D;
 #pragma unroll
-        for (int e = 0; e < kEpl<T>; ++e) x[e] = static_cast<T>(y[e]);
-        u32x4 w;
-        __builtin_memcpy(&w, x, 16);
-        yop[s] = w;
-      } else {
+          for (int j = 0; j < 2; ++j) {
+            const int d0 = qd + j * kScoreWaves * kCols<T>, dc = d0 < D ? d0 : 0;
+            if (qvec) qr[i][j] = *reinterpret_cast<const u32x4*>(qrow[i] + dc);
 #pragma unroll
-        for (int u = 0; u < YV; ++u) {
-          u32x4 w;
-          __builtin_memcpy(&w, y + 4 * u, 16);
-          yop[((rb * nch + c) * YV + u) * 64 + l] = w;
+            for (int u = 0; u < YU; ++u) yr[i][j][u] = *reinterpret_cast<const f32x4*>(yrow + dc + 4 * u);
+          }
         }
-      }
-    }
-    if (tid < R) {
-      const bool in = r0 + tid < M;
-      const int64_t i = ((int64_t)head * mpad + r0 + tid) * 2;
-      row_m[tid] = in ? row_mr[i] : 0.f;
-      row_r[tid] = in ? row_mr[i + 1] : 0.f;
-      yn2[tid] = in ? ystat[i + 1] : 0.f;
-    }
-    __syncthreads();
-    int bound[kRB][4];
-    f32x4 m4[kRB], r4[kRB], y4[kRB];
+        if (r0 == 0 && rb0 == 0 && c0 == 0) load(16 * wv, 0);
 #pragma unroll
-    for (int rb = 0; rb < kRB; ++rb) {
-      m4[rb] = *reinterpret_cast<const f32x4*>(row_m + 16 * rb + 4 * lg);
-      r4[rb] = *reinterpret_cast<const f32x4*>(row_r + 16 * rb + 4 * lg);
-      y4[rb] = *reinterpret_cast<const f32x4*>(yn2 + 16 * rb + 4 * lg);
+        for (int i = 0; i < kRB; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = r0 + 16 * rb + 4 * lg + r;
-        bound[rb][r] = m < M ? Lk - W + m % W - k_begin : -1;  // last visible key, relative to k_begin
-      }
-    }
-
-    for (int t = 16 * wv; t < nrel; t += 16 * kScoreWaves) {
-      f32x4 s[kRB], gg[kRB];
+          for (int j = 0; j < 2; ++j) {
+            const int c = c0 + wv + kScoreWaves * j, ch = (rb0 + i) * nch + c, d0 = qd + j * kScoreWaves * kCols<T>;
+            if (c < nch) {
+              const bool in = r0 + 16 * (rb0 + i) + li < M && d0 < D;
+              if (!qvec) qr[i][j] = gather_unit(qrow[i] + (int64_t)(d0 < D ? d0 : 0) * q_sd, q_sd);
+              qop[ch * 64 + lane] = in ? qr[i][j] : u32x4{0u, 0u, 0u, 0u};
+              f32x4 y[YU];
 #pragma unroll
-      for (int rb = 0; rb < kRB; ++rb) s[rb] = gg[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-      float vsq = 0.f;
-      const uint32_t kr = (uint32_t)(t + li) * kvs.k_rb, vr = (uint32_t)(t + li) * kvs.v_rb;
-      for (int c0 = 0; c0 < nch; c0 += kGrp) {
-        u32x4 kf[kGrp], vf[kGrp];
-#pragma unroll
-        for (int u = 0; u < kGrp; ++u) {
-          const int col = (c0 + u) * kCols<T> + kEpl<T> * lg;
-          const uint32_t cb = col * (uint32_t)sizeof(T);
-          kf[u] = buf_load16(krs, col < D ? kr + cb : kPastAll);
-          vf[u] = buf_load16(vrs, col < D ? vr + cb : kPastAll);
-        }
-#pragma unroll
-        for (int u = 0; u < kGrp; ++u)
-          if (c0 + u < nch) {
-            float ve[kEpl<T>];
-#pragma unroll
-            for (int e = 0; e < kEpl<T>; ++e) {
-              ve[e] = elem_of<T>(vf[u], e);
-              vsq = fmaf(ve[e], ve[e], vsq);
-            }
-#pragma unroll
-            for (int rb = 0; rb < kRB; ++rb) {
-              const int ch = rb * nch + c0 + u;
-              s[rb] = mfma_chunk<T>(qop[ch * 64 + lane], kf[u], s[rb]);
+              for (int u = 0; u < YU; ++u) y[u] = in ? yr[i][j][u] : f32x4{0.f, 0.f, 0.f, 0.f};
               if constexpr (kYT) {
-                gg[rb] = mfma_chunk<T>(yop[ch * 64 + lane], vf[u], gg[rb]);
+                T x[kEpl<T>];
+#pragma unroll
+                for (int e = 0; e < kEpl<T>; ++e) x[e] = static_cast<T>(y[e / 4][e % 4]);
+                u32x4 w;
+                __builtin_memcpy(&w, x, 16);
+                yop[ch * 64 + lane] = w;
               } else {
 #pragma unroll
-                for (int w = 0; w < YV; ++w) {
-                  const f32x4 yf = __builtin_bit_cast(f32x4, yop[(ch * YV + w) * 64 + lane]);
-#pragma unroll
-                  for (int e = 0; e < 4; ++e) gg[rb] = mfma_f32(yf[e], ve[4 * w + e], gg[rb]);
-                }
+                for (int u = 0; u < YU; ++u) yop[(ch * YV + u) * 64 + lane] = __builtin_bit_cast(u32x4, y[u]);
               }
             }
           }
       }
-      const float vn2 = add_xor32(add_xor16(vsq));
-      float sum = 0.f;
+    for (int r = tid; r < 16 * nrb; r += NT) {
+      const bool in = r0 + r < M;
+      const int64_t i = ((int64_t)head * mpad + (in ? r0 + r : 0)) * 2;
+      stf[(r / 16 * 3 + 0) * 16 + r % 16] = in ? row_mr[i] : 0.f;
+      stf[(r / 16 * 3 + 1) * 16 + r % 16] = in ? row_mr[i + 1] : 0.f;
+      stf[(r / 16 * 3 + 2) * 16 + r % 16] = in ? ystat[i + 1] : 0.f;
+    }
+    __syncthreads();
+
+    for (int t = 16 * wv; t < nrel; t += 16 * kScoreWaves) {
+      if (once && (r0 || t != 16 * wv)) load(t, 0);
+      float total = 0.f, vn2 = 0.f;
+      for (int g0 = 0; g0 < nrb; g0 += kRB) {
+        f32x4 s[kRB], gg[kRB];
 #pragma unroll
-      for (int rb = 0; rb < kRB; ++rb)
+        for (int rb = 0; rb < kRB; ++rb) s[rb] = gg[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        float vsq = 0.f;
+        for (int c0 = 0; c0 < nch; c0 += kGrp) {
+          if (!once) load(t, c0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const bool seen = t + li <= bound[rb][r] && t + li < nrel;
-          float p = fminf(__builtin_amdgcn_exp2f((s[rb][r] - m4[rb][r]) * scale_log2) * r4[rb][r], 1.f);
-          if (p_round) p = round_through<T>(p);
-          const float terms = vn2 + y4[rb][r];
-          float d2 = fmaf(-2.f, gg[rb][r], terms);
-          // (NaN counts as cancelled, so that infinite rows give what the
-          // direct form gives.)
-          uint64_t need = __ballot(seen && !(d2 >= kDirect * terms));
-          while (need) {
-            const int l = __builtin_ctzll(need);
-            need &= need - 1;
-            const int key = t + (l & 15), row = 16 * rb + 4 * (l >> 4) + r;
-            const T* vrow = reinterpret_cast<const T*>(vhead + (int64_t)key * kvs.v_rb);
-            const float* yrow = yrow0 + (int64_t)row * D;
-            float a = 0.f;
-            for (int d = lane; d < D; d += 64) {
-              const float x = static_cast<float>(vrow[d]) - yrow[d];
-              a = fmaf(x, x, a);
+          for (int u = 0; u < kGrp; ++u)
+            if (c0 + u < nch) {
+              float ve[kEpl<T>];
+#pragma unroll
+              for (int e = 0; e < kEpl<T>; ++e) ve[e] = elem_of<T>(vf[u], e);
+              if (g0 == 0)
+#pragma unroll
+                for (int e = 0; e < kEpl<T>; ++e) vsq = fmaf(ve[e], ve[e], vsq);
+#pragma unroll
+              for (int rb = 0; rb < kRB; ++rb) {
+                const int ch = (g0 + rb) * nch + c0 + u;
+                s[rb] = mfma_chunk<T>(qop[ch * 64 + lane], kf[u], s[rb]);
+                if constexpr (kYT) {
+                  gg[rb] = mfma_chunk<T>(yop[ch * 64 + lane], vf[u], gg[rb]);
+                } else {
+#pragma unroll
+                  for (int w = 0; w < YV; ++w) {
+                    const f32x4 yf = __builtin_bit_cast(f32x4, yop[(ch * YV + w) * 64 + lane]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) gg[rb] = mfma_f32(yf[e], ve[4 * w + e], gg[rb]);
+                  }
+                }
+              }
             }
-            a = wave_sum_dpp(a);
-            d2 = lane == l ? a : d2;
-          }
-          const float ratio = p / (1.f - p + eps);
-          sum = seen ? fmaf(ratio * ratio, d2, sum) : sum;
         }
-      sum = add_xor16(add_xor32(sum));
+        if (g0 == 0) vn2 = add_xor32(add_xor16(vsq));
+        float sum = 0.f;
+#pragma unroll
+        for (int rb = 0; rb < kRB; ++rb) {
+          const f32x4 m4 = st[(g0 + rb) * 12 + lg], r4 = st[(g0 + rb) * 12 + 4 + lg], y4 = st[(g0 + rb) * 12 + 8 + lg];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int row = 16 * (g0 + rb) + 4 * lg + r, m = r0 + row;
+            const bool seen = m < M && t + li < nrel && k_begin + t + li <= Lk - W + dv.w.mod(m);
+            float p = fminf(__builtin_amdgcn_exp2f((s[rb][r] - m4[r]) * scale_log2) * r4[r], 1.f);
+            if (p_round) p = round_through<T>(p);
+            const float terms = vn2 + y4[r];
+            float d2 = fmaf(-2.f, gg[rb][r], terms);
+            // (NaN counts as cancelled, so that infinite rows give what the
+            // direct form gives.)
+            uint64_t need = __ballot(seen && !(d2 >= kDirect * terms));
+            while (need) {
+              const int l = __builtin_ctzll(need);
+              need &= need - 1;
+              const T* vrow = reinterpret_cast<const T*>(vhead + (int64_t)(t + (l & 15)) * kvs.v_rb);
+              const float* yrow = yrow0 + (int64_t)(16 * (g0 + rb) + 4 * (l >> 4) + r) * D;
+              float a = 0.f;
+              for (int d = lane; d < D; d += 64) {
+                const float x = static_cast<float>(vrow[d]) - yrow[d];
+                a = fmaf(x, x, a);
+              }
+              a = wave_sum_dpp(a);
+              d2 = lane == l ? a : d2;
+            }
+            const float ratio = p / (1.f - p + eps);
+            sum = seen ? fmaf(ratio * ratio, d2, sum) : sum;
+          }
+        }
+        total += sum;
+      }
+      total = add_xor16(add_xor32(total));
       if (lg == 0) {
-        if (r0) sum += sc[t + li];
-        if (r0 + R >= M) {
-          if (t + li < nrel) scores[(int64_t)head * Lk + k_begin + t + li] = sum / inv_g;
+        if (r0) total += sc[t + li];
+        if (r0 + rs >= M) {
+          if (t + li < nrel) scores[(int64_t)head * Lk + k_begin + t + li] = total / static_cast<float>(g);
         } else {
-          sc[t + li] = sum;
+          sc[t + li] = total;
         }
       }
     }
@@ -639,13 +741,16 @@ static hipError_t launch_genm_t(const ScorePlan& p, int D, const void* q, int64_
   const KvStride kvs = kv_strides(kv, sizeof(T));
   const bool flash = sizeof(T) == 4 || !p_round;  // fp32: rounding p is the identity
   const int nch = (D + kCols<T> - 1) / kCols<T>;
-  const int CG = (D + 63) / 64, KG = kPartWaves / CG;
+  const int CG = (D + 63) / 64, KG = part_kg(CG);
+  const ScoreDiv dv{Div::of(p.n_mc), Div::of(p.s1), Div::of(Hkv), Div::of(W)};
   const size_t ops = (size_t)kRB * nch * 64 * 16;
-  const size_t lds1 = std::max(ops + (size_t)16 * kRB * kPPitch * 4, (size_t)KG * 16 * kRB * CG * 64 * 4);
+  const bool qvec = q_sd == 1 && (q_sb * sizeof(T)) % 16 == 0 && (q_sh * sizeof(T)) % 16 == 0 &&
+                    (q_ss * sizeof(T)) % 16 == 0 && (reinterpret_cast<uintptr_t>(q) & 15u) == 0;
+  const size_t lds1 = std::max(ops + (size_t)16 * kRB * kPPitch * 4, (size_t)KG * 16 * kRB * (CG * 64 + 4) * 4);
   const dim3 g1(p.heads * p.n_mc * p.s1), b1(64 * kPartWaves);
   auto part = [&](auto kern, size_t lds) {
-    launch(kern, g1, b1, lds, st, qq, q_sb, q_sh, q_ss, q_sd, kk, vv, kvs, Hkv, Lq, Lk, D, W, p.g, p.M, p.n_mc, p.s1,
-           p.kps1, scale_log2, part_ml, part_y, row_mr);
+    launch(kern, g1, b1, lds, st, qq, q_sb, q_sh, q_ss, q_sd, qvec, kk, vv, kvs, Hkv, Lq, Lk, D, W, p.g, p.M, p.n_mc, p.s1,
+           p.kps1, scale_log2, part_ml, part_y, row_mr, dv);
   };
   if (flash) {
     part(genm_part_kernel<T, kRB, kFlash>, lds1);
@@ -653,7 +758,7 @@ static hipError_t launch_genm_t(const ScorePlan& p, int D, const void* q, int64_
     part(genm_part_kernel<T, kRB, kStats>, ops);
     part(genm_part_kernel<T, kRB, kSum>, lds1);
   }
-  launch(genm_merge_kernel<T>, dim3(p.heads * p.M), dim3(64), 0, st, part_ml, part_y, p.n_mc, p.s1, p.M, D,
+  launch(genm_merge_kernel<T>, dim3(p.M, p.heads), dim3(64), 0, st, part_ml, part_y, p.n_mc, p.s1, p.M, D,
          scale_log2, flash ? 1 : 0, y_round, ystat, yf, row_mr, zero_ptr, zero_words);
   // Keys per workgroup: 64 (16 per wave) until there are more workgroups than
   // the GPU runs at once, then more, so that staging Q and Y is shared.
@@ -661,10 +766,15 @@ static hipError_t launch_genm_t(const ScorePlan& p, int D, const void* q, int64_
   const int steps = (Lk + kStep - 1) / kStep;
   const int per = std::min(16, std::max(1, (int)(((int64_t)p.heads * steps + 1023) / 1024)));
   const int kpw = per * kStep, wgs = (Lk + kpw - 1) / kpw;
+  // Rows staged together: all, up to half of the CU's LDS.
+  constexpr size_t kStageBytes = 80 * 1024;
   auto score = [&](auto kern, size_t yv) {
-    launch(kern, dim3(p.heads * wgs), dim3(64 * kScoreWaves), ops * (1 + yv) + (size_t)kpw * 4, st, qq, q_sb, q_sh,
-           q_ss, q_sd, kk, vv, kvs, Hkv, Lq, Lk, D, W, p.g, p.M, p.mpad, scale_log2, eps, p_round, wgs, kpw, ystat,
-           yf, row_mr, scores);
+    const size_t per_group = ops * (1 + yv) + 16 * kRB * 12;
+    const int groups = (p.M + 16 * kRB - 1) / (16 * kRB);
+    const int rs = 16 * kRB * (int)std::max<size_t>(1, std::min<size_t>(groups, kStageBytes / per_group));
+    launch(kern, dim3(p.heads * wgs), dim3(64 * kScoreWaves), per_group * (rs / (16 * kRB)) + (size_t)kpw * 4, st, qq,
+           q_sb, q_sh, q_ss, q_sd, qvec, kk, vv, kvs, Hkv, Lq, Lk, D, W, p.g, p.M, p.mpad, scale_log2, eps, p_round,
+           kpw, rs, ystat, yf, row_mr, scores, ScoreDiv{dv.n_mc, Div::of(wgs), dv.hkv, dv.w});
   };
   if constexpr (sizeof(T) == 2) {
     if (y_round)
