@@ -250,7 +250,8 @@ static int evict_impl(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, i
   if (rc) return rc;
   if (!k_out || !v_out) return fail(DROPKV_E_ARG, "null k_out/v_out pointer");
   if (out_ld < keep) return fail(DROPKV_E_ARG, "row capacity below the rows used");
-  const dkv::ScorePlan p = dkv::make_score_plan(B, Hq, Hkv, Lk, D, W, splits);
+  dkv::ScorePlan p = dkv::make_score_plan(B, Hq, Hkv, Lk, D, W, splits);
+  if (splits <= 0) dkv::plan_solo_rows(&p, Lk);
   const size_t s_bytes = ((size_t)B * Hkv * Lk * 4 + 255) & ~size_t(255);
   const size_t need = p.total + s_bytes + dkv::select_workspace_bytes(B * Hkv, Lk);
   if (!workspace || workspace_bytes < need)

@@ -56,6 +56,9 @@ struct ScorePlan {
 };
 
 ScorePlan make_score_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Lk, int64_t D, int64_t W, int64_t splits);
+// A layer-call of short rows: one pass-2 workgroup per row (plan_solo_rows
+// changes the plan where that is the faster split).
+void plan_solo_rows(ScorePlan* p, int64_t Lk);
 struct SelectCompact;
 // Pooling fused into the scoring pass: the selection workspace (its per-row
 // words are cleared by the merge kernel through zero_ptr) and the pooling

@@ -799,7 +799,10 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs,
   if (fz.enabled) {
     __syncthreads();  // this workgroup's score stores are done; the LDS operands are dead
     if (fz.full) {
-      fused_tail<NT>(fz, sc_row, hist_l, head, split, n_splits, kps, Lk);
+      if (n_splits == 1)
+        solo_tail<NT>(fz, sc_row, hist_l, head, kps, Lk);
+      else
+        fused_tail<NT>(fz, sc_row, hist_l, head, split, n_splits, kps, Lk);
       return;
     }
     const int h = fz.ks / 2;
@@ -1200,6 +1203,20 @@ bool kv_rows_fit(int64_t row_stride, int64_t elem_bytes, int64_t Lk, int64_t D) 
 KvStride kv_strides(const KvSrc& kv, int64_t elem_bytes) {
   return KvStride{kv.k_sb, kv.k_sh, kv.v_sb, kv.v_sh, (uint32_t)(kv.k_sl * elem_bytes),
                   (uint32_t)(kv.v_sl * elem_bytes)};
+}
+
+// Rows of up to two tiles for each of pass 2's eight waves are left to one
+// workgroup each: the second tile costs ~2 us, the selection among several
+// workgroups ~7 us more than within one (layer-call, us, one workgroup per row
+// against Lk / 256: 512 keys, 8 / 2 heads of 64: 25.3 and 30.9, 32 / 8 of 128:
+// 32.7 and 35.9, 3 x 28 / 4 of 128: 36.4 and 39.2; with three or four tiles a
+// wave, 800 keys: 30.3 and 32.4, 38.9 and 37.8, 43.0 and 41.2).
+constexpr int kSoloKeys = 512;
+void plan_solo_rows(ScorePlan* p, int64_t Lk) {
+  static_assert(kSoloKeys <= kScLds, "a row's scores in LDS");
+  if (p->p1_wide || p->n_mc > 2 || Lk > kSoloKeys) return;
+  p->kps2 = ceil_div(Lk, kTile) * kTile;
+  p->s2 = 1;
 }
 
 namespace {

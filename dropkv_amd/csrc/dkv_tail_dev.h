@@ -301,6 +301,97 @@ __device__ __forceinline__ void tail_emit(const SelFuse& fz, int row, int j0, in
   }
 }
 
+// The whole selection of one row whose scores one workgroup holds (sc, n =
+// Lk keys): the same rule as fused_tail with everything in LDS, so no
+// barriers between workgroups and nothing published.  The candidates (keys
+// inside the top-digit bin of the keep-th key) of a row this short are few:
+// up to kSoloRank of them are ranked against each other at once (a group of
+// threads per candidate), without a second digit.  Pass 2 of a 512-key layer-call
+// (2 rows, D = 64): 17.6 us in two workgroups per row with fused_tail, 11.9 in
+// one with this; 300 keys, one workgroup either way: 17.4 and 11.6.  L: tail_lds_words(NT, kps)
+// words of LDS (pass 2's operands are dead).
+constexpr uint32_t kSoloRank = 128;
+
+template <int NT>
+__device__ void solo_tail(const SelFuse& fz, const float* __restrict__ sc, uint32_t* L, int row, int kps, int Lk) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int h = fz.ks / 2, prot = Lk - fz.window;
+  uint32_t* hist1 = L;
+  uint32_t* small = hist1 + kBins1;  // [0, 32) block scans, [64, 72) bin searches, 124 candidates, 127 max
+  float* pl = reinterpret_cast<float*>(small + 128);
+  uint32_t* U = small + 128 + ((kps + 3) & ~3);  // candidates' keys, then emit slots
+  uint32_t* hist2 = U + tail_u_words(NT);
+  uint32_t* hist3 = hist2 + kBins2;
+  for (int i = tid; i < kBins1; i += NT) hist1[i] = 0u;
+  if (tid == 0) {
+    small[124] = 0u;
+    small[127] = 0u;
+  }
+  __syncthreads();
+  uint32_t kmax = 0u;
+  for (int j = tid; j < Lk; j += NT) {
+    const float m = lds_window_max(sc, max(j - h, 0), min(j + h, Lk - 1));
+    pl[j] = m;
+    const uint32_t key = float_key(m);
+    kmax = max(kmax, key);
+    if (j < prot) atomicAdd(&hist1[key >> kShift1], 1u);
+  }
+  kmax = wave_reduce_max(kmax);
+  if (lane == 0 && kmax) atomicMax(&small[127], kmax);
+  __syncthreads();
+  const uint32_t kbig = float_key(key_float(small[127]) + 1.0f);
+  if (tid < 64) {
+    // (one wave: its own LDS operations stay in order)
+    if (tid == 0) hist1[kbig >> kShift1] += (uint32_t)fz.window;
+    wave_find_bin<kBins1>(hist1, nullptr, (uint32_t)fz.keep, small + 64);
+  } else {
+    for (int i = tid - 64; i < kBins2 + kBins3; i += NT - 64) hist2[i] = 0u;  // (hist3 follows)
+  }
+  __syncthreads();
+  const uint32_t b1 = small[64], k1 = (uint32_t)fz.keep - small[65];
+  const uint32_t m = hist1[b1];  // candidates
+  auto key_of = [&](int j) { return j >= prot ? kbig : float_key(pl[j]); };
+  auto for_cands = [&](auto&& f) __attribute__((always_inline)) {
+    for (int j = tid; j < Lk; j += NT) {
+      const uint32_t key = key_of(j);
+      if ((key >> kShift1) == b1) f(key, j);
+    }
+  };
+  uint32_t T, take_eq;
+  if (m <= kSoloRank) {
+    for_cands([&](uint32_t key, int) { U[atomicAdd(&small[124], 1u)] = key; });
+    __syncthreads();
+    // NT / kSoloRank threads (of one wave) per candidate.
+    constexpr int kGroup = NT / (int)kSoloRank;
+    static_assert(kGroup >= 1 && kGroup <= 64 && (kGroup & (kGroup - 1)) == 0, "a group of lanes per candidate");
+    const uint32_t c = tid / kGroup;
+    const uint32_t mine = c < m ? U[c] : 0u;
+    uint32_t above = 0u, same = 0u;
+    for (uint32_t i = tid % kGroup; i < m; i += kGroup) {
+      const uint32_t o = U[i];
+      above += o > mine ? 1u : 0u;
+      same += o == mine ? 1u : 0u;
+    }
+#pragma unroll
+    for (int o = 1; o < kGroup; o <<= 1) {
+      above += __shfl_xor(above, o);
+      same += __shfl_xor(same, o);
+    }
+    if (c < m && above < k1 && k1 <= above + same) {  // (equal candidates write the same)
+      small[68] = mine;
+      small[69] = k1 - above;
+    }
+    __syncthreads();
+    T = small[68];
+    take_eq = small[69];
+  } else {
+    tail_digits(for_cands, b1, k1, hist2, hist3, small + 64, &T, &take_eq);
+  }
+  int* s_src = reinterpret_cast<int*>(U);
+  tail_emit<NT>(fz, row, 0, Lk, 0u, 0u, T, take_eq, kbig, prot, [&](int j) { return pl[j]; }, s_src,
+                s_src + NT * kEmitPer, small);
+}
+
 // The whole selection of one row by the pass-2 workgroup of split `split`
 // (keys [split*kps, min((split+1)*kps, Lk))) once its scores are in LDS (sc).
 // L: tail_lds_words(NT, kps) words of LDS (pass 2's operands are dead).
