@@ -228,15 +228,21 @@ def append(K: torch.Tensor, V: torch.Tensor, k_buf: torch.Tensor, v_buf: torch.T
     dev = _check_device(K, V, k_buf, v_buf)
     _check_buffer(k_buf, "k_buf")
     _check_buffer(v_buf, "v_buf")
-    if K.shape != V.shape or K.dtype != V.dtype or k_buf.shape != v_buf.shape:
+    # (Shapes and strides read once: this call runs per layer and chunk, and
+    # its host time is of the order of the copy's.)
+    shape, bshape, dtype = K.shape, k_buf.shape, K.dtype
+    if shape != V.shape or dtype != V.dtype or bshape != v_buf.shape:
         raise RuntimeError("K/V and the buffers must match in shape and dtype")
-    if K.dtype != k_buf.dtype or K.shape[:2] != k_buf.shape[:2] or K.shape[3] != k_buf.shape[3]:
+    B, H, L, D = shape
+    bB, bH, C, bD = bshape
+    if dtype != k_buf.dtype or B != bB or H != bH or D != bD:
         raise RuntimeError("K/V do not fit the buffers")
-    if K.stride(3) != 1 or V.stride(3) != 1 or K.stride() != V.stride():
+    strides = K.stride()
+    if strides[3] != 1 or strides != V.stride():
         K, V = K.contiguous(), V.contiguous()
-    B, H, L, D = K.shape
-    rc = _lib.load().dropkv_append(K.data_ptr(), V.data_ptr(), *_seg_strides(K), K.element_size(), B, H, L, D,
-                                   k_buf.data_ptr(), v_buf.data_ptr(), k_buf.shape[2], int(row0), _stream(dev))
+        strides = K.stride()
+    rc = _lib.load().dropkv_append(K.data_ptr(), V.data_ptr(), strides[0], strides[1], strides[2], K.element_size(),
+                                   B, H, L, D, k_buf.data_ptr(), v_buf.data_ptr(), C, int(row0), _stream(dev))
     _lib.check(rc, "dropkv_append")
 
 
