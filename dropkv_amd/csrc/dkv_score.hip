@@ -80,14 +80,6 @@ pass1_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, 
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4;
 
-  v8 qop[kMB][KK];
-  int bound[kMB];
-#pragma unroll
-  for (int mb = 0; mb < kMB; ++mb) {
-    const int m = mc * kRows + mb * 16 + li;
-    load_q_ops<T, D>(qop[mb], q, q_sb, q_sh, q_ss, q_sd, qvec, b, hkv, g, W, Lq, M, m, lg);
-    bound[mb] = row_bound(m, M, W, Lk);
-  }
   // Tiles wholly below every row's causal bound need no masking (unless this
   // chunk holds padding rows).
   const bool pad_chunk = mc * kRows + kRows > M;
@@ -109,6 +101,20 @@ pass1_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, 
     for (int i = 0; i < NVC; ++i) vc[i] = buf_load16(vrs, base + (uint32_t)(i * GRP) * kvs.v_rb);
   };
 
+  // The wave's first tile on its way before the query rows are addressed: the
+  // kernel is bound by its K/V stream, which used to start only after the
+  // query rows' address arithmetic (the wait for the rows now also waits for
+  // the tile, but their latencies are the same one).  B=1 Hq=32 Hkv=8 D=128
+  // W=8 at Lk 32768: 33.4 -> 32.4 us.
+  v8 kop[2][KK];
+  u32x4 vch[NVC];
+  load_rows_op<T, D>(kop, krs, k_lane, wv * kTile, kvs.k_rb);  // zeros past the split's end
+  load_v(vch, wv * kTile);
+  v8 qop[kMB][KK];
+  load_q_ops<T, D>(qop, q, q_sb, q_sh, q_ss, q_sd, qvec, b, hkv, g, W, Lq, M, mc * kRows, li, lg);
+  int bound[kMB];
+#pragma unroll
+  for (int mb = 0; mb < kMB; ++mb) bound[mb] = row_bound(mc * kRows + mb * 16 + li, M, W, Lk);
   float m2[kMB], lsum[kMB];
   // Per lane: the largest logit among its own keys and the lowest key
   // holding it (-1: none yet).
@@ -125,8 +131,6 @@ pass1_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, 
     for (int dt = 0; dt < DT; ++dt) yacc[dt][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  v8 kop[2][KK];
-  u32x4 vch[NVC];
   const int stride = WAVES * kTile;
 
   // One tile (t0 absolute, tn relative to k_begin): consume the K/V
@@ -196,8 +200,6 @@ pass1_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss, 
   // order, and so every bit of the result, is the same on every call.
   const int nrel = k_end - k_begin;
   int t = wv * kTile;  // relative to k_begin
-  load_rows_op<T, D>(kop, krs, k_lane, t, kvs.k_rb);  // zeros if t >= nrel
-  load_v(vch, t);
   for (; t < nrel; t += stride) tile(kop, vch, k_begin + t, t + stride);
 
   // Row sums are per lane-group partials; fold the four groups.  The lanes'
@@ -340,7 +342,9 @@ pass1w_kernel(const T* __restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_ss,
 #pragma unroll
   for (int mb = 0; mb < kMB; ++mb) {
     const int m = mc * kRows + mb * 16 + li;
-    load_q_ops<T, D>(qop[mb], q, q_sb, q_sh, q_ss, q_sd, qvec, b, hkv, g, W, Lq, M, m, lg);
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+      qop[mb][kk] = load_q_op<T>(q, q_sb, q_sh, q_ss, q_sd, qvec, b, hkv, g, W, Lq, M, m, 32 * kk + 8 * lg);
     bound[mb] = row_bound(m, M, W, Lk);
   }
   const bool pad_chunk = mc * kRows + kRows > M;
@@ -549,7 +553,7 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs,
              int Hkv, int Lq, int Lk, int W, int g, int M, int n_mc, int cg, int n_splits, int kps,
              float scale_log2, float eps, float small_c2,
              const u32x4* __restrict__ opblk, const float* __restrict__ stblk, float* __restrict__ scores,
-             SelFuse fz) {
+             SelFuse fz, Div d_splits, Div d_hkv) {
   typedef typename Elem<T>::v8 v8;
   constexpr int KK = D / 32;
   constexpr int OPS = kOpSlots * kMB * KK;  // operand slots per row-chunk (Q, Yhi, Ylo)
@@ -578,12 +582,33 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs,
   DKV_ARG_NOW(n_mc);
   DKV_ARG_NOW(cg);
   DKV_ARG_NOW(g);
+  DKV_ARG_NOW(d_splits.m);
+  DKV_ARG_NOW(d_splits.s);
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int split = lid % n_splits;
-  const int head = lid / n_splits;
-  const int b = head / Hkv, hkv = head % Hkv;
+  const int head = d_splits.div(lid), split = lid - head * n_splits;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4;
+
+  // Operands of row-chunks c0 .. c0+cn-1 (written by the merge kernel in
+  // LDS order).  Those of the first group are asked for before anything else
+  // is worked out: the kernel cannot start on its first tile without them
+  // (B=1 Hq=32 Hkv=8 D=128 W=8 at Lk 32768, update: 81.6 -> 81.0 us; B=2 at
+  // Lk 7001: 70.6 -> 69.8).
+  constexpr int SPW = (2 * OPS * 64 + NT - 1) / NT;
+  static_assert(4 * kMB * kStatWords <= NT, "one statistics word per thread");
+  u32x4 sv[SPW];
+  float stv;
+  auto load_ops = [&](int c0, int cn) __attribute__((always_inline)) {
+    const int nw = cn * OPS * 64, ns = cn * kMB * kStatWords;
+    const u32x4* gop = opblk + ((size_t)head * n_mc + c0) * OPS * 64;
+    const float* gst = stblk + ((size_t)head * n_mc + c0) * kMB * kStatWords;
+#pragma unroll
+    for (int i = 0; i < SPW; ++i) sv[i] = gop[min((int)threadIdx.x + i * NT, nw - 1)];
+    stv = gst[min((int)threadIdx.x, ns - 1)];
+  };
+  load_ops(0, min(cg, n_mc));
+  __builtin_amdgcn_sched_barrier(0);
+  const int b = d_hkv.div(head), hkv = head - b * Hkv;
 
   // The per-key sums hold sum_m w * (-dist2/2): scale by -2/g at the end.
   const float out_scale = -2.0f * (1.0f / static_cast<float>(g));
@@ -600,22 +625,13 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs,
   for (int c0 = 0; c0 < n_mc; c0 += cg) {
     const int cn = min(cg, n_mc - c0);
     const bool first = c0 == 0, last = c0 + cn >= n_mc;
-    // Operands of row-chunks c0 .. c0+cn-1 (written by the merge kernel in
-    // LDS order): issue their loads, then the first tile's K/V loads, so both
-    // round trips overlap; the LDS writes wait only for the former.  Every
-    // wave issues its operand loads before any wave issues K/V loads (the
-    // barrier between them): otherwise the later waves' operand loads queue
-    // behind the earlier waves' 16 KB of K/V each, and the operand block
-    // reaches LDS ~2 us later.
-    constexpr int SPW = (2 * OPS * 64 + NT - 1) / NT;
+    // The operands' loads, then the first tile's K/V loads, so both round trips
+    // overlap; the LDS writes wait only for the former.  Every wave issues its
+    // operand loads before any wave issues K/V loads (the barrier between
+    // them): otherwise the later waves' operand loads queue behind the earlier
+    // waves' 16 KB of K/V each, and the operand block reaches LDS ~2 us later.
     const int nw = cn * OPS * 64, ns = cn * kMB * kStatWords;
-    static_assert(4 * kMB * kStatWords <= NT, "one statistics word per thread");
-    const u32x4* gop = opblk + ((size_t)head * n_mc + c0) * OPS * 64;
-    const float* gst = stblk + ((size_t)head * n_mc + c0) * kMB * kStatWords;
-    u32x4 sv[SPW];
-#pragma unroll
-    for (int i = 0; i < SPW; ++i) sv[i] = gop[min((int)threadIdx.x + i * NT, nw - 1)];
-    const float stv = gst[min((int)threadIdx.x, ns - 1)];
+    if (!first) load_ops(c0, cn);
     // Tiles are handed out dynamically: wave w starts with tile w, then
     // takes the next unclaimed one from s_next (relative to k_begin).  Each
     // key's score is computed by one wave in a fixed order, so the results do
@@ -632,7 +648,8 @@ pass2_kernel(const T* __restrict__ kp, const T* __restrict__ vp, KvStride kvs,
     for (int i = 0; i < SPW; ++i)
       if ((int)threadIdx.x + i * NT < nw) opnd[threadIdx.x + i * NT] = sv[i];
     // Groups of four row-chunks copy the second pair directly.
-    for (int i = SPW * NT + (int)threadIdx.x; i < nw; i += NT) opnd[i] = gop[i];
+    for (int i = SPW * NT + (int)threadIdx.x; i < nw; i += NT)
+      opnd[i] = opblk[((size_t)head * n_mc + c0) * OPS * 64 + i];
     if ((int)threadIdx.x < ns) stat[threadIdx.x] = stv;
     __syncthreads();
 
@@ -1353,7 +1370,7 @@ static hipError_t launch_scores_t(const ScorePlan& p, const void* q, int64_t q_s
     }
   }
   launch(k2, g2, dim3(512), lds2, st, kk, vv, kvs, Hkv, Lq, Lk, W, p.g, p.M, p.n_mc, cg, p.s2, p.kps2, scale_log2,
-         eps, small_c2, opblk, stblk, scores, fz);
+         eps, small_c2, opblk, stblk, scores, fz, Div::of(p.s2), Div::of(Hkv));
   return hipGetLastError();
 }
 

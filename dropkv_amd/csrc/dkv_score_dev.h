@@ -148,14 +148,47 @@ __device__ __forceinline__ typename Elem<T>::v8 load_q_op(const T* __restrict__ 
   return x;
 }
 
-// Load the Q^T operands of one 16-row block (lane row m, lane group lg).
+// The Q^T operands of kMB 16-row blocks from row m0 (lane row m0 + 16 mb + li,
+// lane group lg: columns 32 kk + 8 lg .. +7; zeros for padding rows).  With
+// `qvec` (head-dim stride 1 and 16-byte aligned rows, checked by the host)
+// 16-byte loads, all issued in a row; otherwise element loads, so Q may have
+// any strides.
 template <typename T, int D>
-__device__ __forceinline__ void load_q_ops(typename Elem<T>::v8 (&qop)[D / 32], const T* __restrict__ q,
+__device__ __forceinline__ void load_q_ops(typename Elem<T>::v8 (&qop)[kMB][D / 32], const T* __restrict__ q,
                                            int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd, bool qvec,
-                                           int b, int hkv, int g, int W, int Lq, int M, int m, int lg) {
+                                           int b, int hkv, int g, int W, int Lq, int M, int m0, int li, int lg) {
+  typedef typename Elem<T>::v8 v8;
+  const T* row[kMB];
 #pragma unroll
-  for (int kk = 0; kk < D / 32; ++kk)
-    qop[kk] = load_q_op<T>(q, q_sb, q_sh, q_ss, q_sd, qvec, b, hkv, g, W, Lq, M, m, 32 * kk + 8 * lg);
+  for (int mb = 0; mb < kMB; ++mb) {
+    const int m = m0 + 16 * mb + li, mm = m < M ? m : 0;  // padding rows read row 0, then zero it
+    const int gi = mm / W, w = mm - gi * W;
+    row[mb] = q + (int64_t)b * q_sb + (int64_t)(hkv * g + gi) * q_sh + (int64_t)(Lq - W + w) * q_ss;
+  }
+  if (qvec) {
+#pragma unroll
+    for (int mb = 0; mb < kMB; ++mb)
+#pragma unroll
+      for (int kk = 0; kk < D / 32; ++kk) qop[mb][kk] = *reinterpret_cast<const v8*>(row[mb] + 32 * kk + 8 * lg);
+  } else {
+#pragma unroll
+    for (int mb = 0; mb < kMB; ++mb)
+#pragma unroll 1
+      for (int kk = 0; kk < D / 32; ++kk) {
+        v8 x;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = row[mb][(int64_t)(32 * kk + 8 * lg + e) * q_sd];
+#pragma unroll
+        for (int j = 0; j < D / 32; ++j)
+          if (j == kk) qop[mb][j] = x;
+      }
+  }
+  if (m0 + 16 * kMB > M)
+#pragma unroll
+    for (int mb = 0; mb < kMB; ++mb)
+      if (m0 + 16 * mb + li >= M)
+#pragma unroll
+        for (int kk = 0; kk < D / 32; ++kk) qop[mb][kk] = v8{};
 }
 
 // Next tile for this wave from the workgroup's LDS counter: waves that get
