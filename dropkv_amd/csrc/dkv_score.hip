@@ -1179,8 +1179,17 @@ ScorePlan make_score_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Lk, int64_
   // splits per head, 75.3 us per layer-call against 76.9 us with 32).  A
   // small call is latency-bound and keeps one workgroup per CU.
   const bool p1_bw = (int64_t)p.heads * Lk * D * 2 * 2 >= (int64_t(32) << 20);
+  // With two row-chunks the same stream is read twice, the second time from
+  // the caches, and is bound by the arithmetic: there every CU gets a
+  // workgroup (no second, nearly empty wave of them: rounded down), as long as
+  // the merge still combines at most kMergeFew partials in one round (D=128,
+  // W=16, B=2 Hkv=8 at Lk 32768: 177 -> 154 us per layer-call; B=1 at 16384:
+  // 61.7 -> 57.3; B=5 at 8192: 125 -> 111; B=12 at 3001: the same).
+  constexpr int kMergeFew = 64;
   const int target1 = (p1_bw && !p.p1_wide) ? DKV_TARGET_P1_BW : target;
   int s1 = splits > 0 ? (int)splits : ceil_div(target1, p1_groups);
+  if (splits <= 0 && p1_bw && !p.p1_wide && p.n_mc > 1)
+    s1 = max(s1, min(kMergeFew, (int)(target / p1_groups)));
   s1 = max(1, min(min(s1, max_by_work), kMaxSplits));
   p.kps1 = ceil_div(ceil_div(Lk, s1), kTile) * kTile;
   p.s1 = ceil_div(Lk, p.kps1);
