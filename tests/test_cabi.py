@@ -173,3 +173,17 @@ def test_noalloc_limits_in_the_header_match_the_library(lib):
     c5 = lib.dropkv_evict_workspace_bytes(4, 64, 8, 131072, 128, 32, 0) / 2 ** 20
     assert abs(float(m.group(3)) - c5) < 0.05
     assert c5 * 2 ** 20 > _lib.NOALLOC_SCRATCH_BYTES
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,W,few", [(1, 32, 8, 128, 16, 10), (2, 32, 8, 128, 16, 5), (1, 14, 2, 64, 8, 40)])
+def test_filling_pass1_leaves_the_noalloc_limit(lib, B, Hq, Hkv, D, W, few):
+    """Two row-chunks: pass 1's split count fills the GPU, up to 2^20 keys in
+    all.  There the scratch is larger than with the few splits of a
+    one-chunk call and far below the static scratch; beyond, it is the same,
+    so no call that the static scratch holds is refused for it."""
+    def need(Lk, splits):
+        return lib.dropkv_evict_workspace_bytes(B, Hq, Hkv, Lk, D, W, splits)
+
+    edge = (1 << 20) // (B * Hkv)
+    assert need(edge, few) < need(edge, 0) < _lib.NOALLOC_SCRATCH_BYTES * 3 // 4
+    assert need(edge + 1, 0) == need(edge + 1, few)
