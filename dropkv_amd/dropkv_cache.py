@@ -219,9 +219,9 @@ class DropKVCache(_LayerCache):
     def _fast_path_ok(self, query_states, key_states, value_states) -> bool:
         """Whether ``dropkv_scores_triton`` accepts these inputs (its
         ``AssertionError`` guards, dropkv_triton.py:680-716); K/V count as
-        contiguous because the fused call makes them so, as
-        ``_compute_keep_indices`` passes ``.contiguous()`` copies
-        (dropkv_cache.py:392-398)."""
+        contiguous because the fused call reads them by their strides (or
+        copies them), as ``_compute_keep_indices`` passes ``.contiguous()``
+        copies (dropkv_cache.py:392-398)."""
         if not self.use_triton:
             return False
         try:
