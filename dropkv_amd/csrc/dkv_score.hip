@@ -1185,14 +1185,17 @@ ScorePlan make_score_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Lk, int64_
   // the merge still combines at most kMergeFew partials in one round (D=128,
   // W=16, B=2 Hkv=8 at Lk 32768: 177 -> 154 us per layer-call; B=1 at 16384:
   // 61.7 -> 57.3; B=5 at 8192: 125 -> 111; B=12 at 3001: the same).
-  // Up to 2^20 keys in all: the extra partials (2 MB at most) must not push a
-  // call that fits the 32 MiB of the no-allocation entry point over them, and
-  // far below that limit (16 MB of scratch at 2^20 keys) they cannot.
+  // Up to 2^20 keys in all: the extra partials must not push a call that fits
+  // the 32 MiB of the no-allocation entry point over them.  At the tuned head
+  // dimensions they are 2 MB at most, and the scratch 29 MB with them.  The
+  // partials grow with D: with the rule at every D, calls of D = 256 to 1024
+  // that the entry point takes were refused (B=1 Hq=32 Hkv=8 D=1024 W=16 at Lk
+  // 4096: 26.4 -> 38.5 MiB), and above D = 256 no kernel reads them.
   constexpr int kMergeFew = 64;
   constexpr int64_t kFillKeys = int64_t(1) << 20;
   const int target1 = (p1_bw && !p.p1_wide) ? DKV_TARGET_P1_BW : target;
   int s1 = splits > 0 ? (int)splits : ceil_div(target1, p1_groups);
-  if (splits <= 0 && p1_bw && !p.p1_wide && p.n_mc > 1 && p.heads * Lk <= kFillKeys)
+  if (splits <= 0 && p1_bw && !p.p1_wide && p.n_mc > 1 && mfma_head_dim(D) && p.heads * Lk <= kFillKeys)
     s1 = max(s1, min(kMergeFew, (int)(target / p1_groups)));
   s1 = max(1, min(min(s1, max_by_work), kMaxSplits));
   p.kps1 = ceil_div(ceil_div(Lk, s1), kTile) * kTile;

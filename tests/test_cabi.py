@@ -187,3 +187,24 @@ def test_filling_pass1_leaves_the_noalloc_limit(lib, B, Hq, Hkv, D, W, few):
     edge = (1 << 20) // (B * Hkv)
     assert need(edge, few) < need(edge, 0) < _lib.NOALLOC_SCRATCH_BYTES * 3 // 4
     assert need(edge + 1, 0) == need(edge + 1, few)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,W", [(1, 32, 8, 16), (2, 32, 8, 16), (1, 14, 2, 8), (20, 32, 2, 4)])
+@pytest.mark.parametrize("D", [96, 192, 256, 512, 768, 1024, 4096])
+def test_other_head_dims_keep_pass1s_few_splits(lib, B, Hq, Hkv, W, D):
+    """The partials grow with D, so at head dimensions outside the tuned ones
+    filling the GPU with splits would push calls over the static scratch:
+    there a bandwidth-bound call has the splits of one that leaves CUs idle
+    (160 workgroups of pass 1), at every length."""
+    groups = B * Hkv * -(-Hq // Hkv * W // 32)
+    for Lk in (2048, 4096, 8192, 24390, 32768, 65536):
+        if groups > 64 or B * Hkv * Lk * D * 4 < 32 << 20:
+            continue
+        few = lib.dropkv_evict_workspace_bytes(B, Hq, Hkv, Lk, D, W, -(-160 // groups))
+        assert lib.dropkv_evict_workspace_bytes(B, Hq, Hkv, Lk, D, W, 0) == few, Lk
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,W,Lk", [(1, 32, 8, 1024, 16, 4096), (1, 14, 2, 1024, 8, 32768),
+                                             (2, 32, 8, 768, 16, 2048), (20, 32, 2, 256, 4, 24390)])
+def test_noalloc_scratch_holds_large_head_dims(lib, B, Hq, Hkv, D, W, Lk):
+    assert 0 < lib.dropkv_evict_workspace_bytes(B, Hq, Hkv, Lk, D, W, 0) <= _lib.NOALLOC_SCRATCH_BYTES
