@@ -319,8 +319,13 @@ static DecodeSplits decode_splits(int64_t heads, int C) {
   return DecodeSplits{(tiles + per - 1) / per, per * kDecTile};
 }
 
+// For the most splits that decode_splits gives any number of heads (two tiles a
+// split at least), so that the size grows with the batch and the capacity: a
+// workspace for the largest call holds every smaller one, whose splits may be
+// more.
 size_t decode_workspace_bytes(int B, int Hq, int Hkv, int D, int C) {
-  const size_t S = (size_t)decode_splits((int64_t)B * Hkv, C).S;
+  const size_t tiles = ((size_t)C + kDecTile - 1) / kDecTile;
+  const size_t S = std::min<size_t>(kDecMaxSplits, (tiles + kDecMinTiles - 1) / kDecMinTiles);
   const size_t rows = (size_t)B * Hkv * S * (Hq / Hkv);
   return rows * sizeof(float) * (2 + (size_t)D) + 256;
 }

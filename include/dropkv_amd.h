@@ -294,7 +294,9 @@ int dropkv_selftest_mfma(float* out, void* stream);
  * caller adds 1 after the step (so a captured graph replays every step).
  * Requires *n_rows < capacity; larger values are clamped to capacity - 1 and
  * overwrite the last row.  Hq / Hkv <= 16, D in dropkv_supported_head_dims.
- * The workspace (dropkv_decode_workspace_bytes) holds the split partials.
+ * The workspace (dropkv_decode_workspace_bytes) holds the split partials; its
+ * size does not fall as B or capacity grow, so one sized for the largest call
+ * holds every smaller one.
  * ------------------------------------------------------------------------ */
 size_t dropkv_decode_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t capacity);
 int dropkv_decode_attention(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sd, const void* k_new,

@@ -208,3 +208,18 @@ def test_other_head_dims_keep_pass1s_few_splits(lib, B, Hq, Hkv, W, D):
                                              (2, 32, 8, 768, 16, 2048), (20, 32, 2, 256, 4, 24390)])
 def test_noalloc_scratch_holds_large_head_dims(lib, B, Hq, Hkv, D, W, Lk):
     assert 0 < lib.dropkv_evict_workspace_bytes(B, Hq, Hkv, Lk, D, W, 0) <= _lib.NOALLOC_SCRATCH_BYTES
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (14, 2, 64), (16, 1, 128)])
+def test_decode_workspace_holds_every_smaller_call(lib, Hq, Hkv, D):
+    """A program sizes one decode workspace for its largest batch and longest
+    cache: the size must not be larger for a smaller one (it is checked on
+    every call)."""
+    caps = [1, 31, 32, 33, 63, 64, 65, 96, 127, 128, 1000, 2048, 4095, 4096, 4097, 4128, 4160, 8192, 100001]
+    sizes = [[lib.dropkv_decode_workspace_bytes(B, Hq, Hkv, D, C) for C in caps]
+             for B in (1, 2, 3, 7, 8, 32, 33, 64, 65, 257)]
+    assert sizes[0][0] > 0
+    for row in sizes:
+        assert row == sorted(row)
+    for small, large in zip(sizes, sizes[1:]):
+        assert all(a <= b for a, b in zip(small, large))
