@@ -306,15 +306,25 @@ __global__ void __launch_bounds__(64) decode_merge_kernel(DecodeArgs a) {
 // with 1024, 56.1 with 2048), two tiles a split at least (a short cache of 1639
 // rows, 2 heads, D = 64: 7.0 us a layer, against 8.7 with one tile a split and
 // 7.7 with four).
+// Where the heads do not divide the 512 waves, rounding down leaves some out.
+// At D = 128 (16 KB in flight a wave) that costs less than the last, partly
+// filled wave of rounding up (171 heads of 8128 rows: 124 us with 2 splits, 143
+// with 3; 257 heads: 215 with 1, 219 with 2).  At D = 64 a wave has only 8 KB in
+// flight, and with a sixteenth of the waves missing or more rounding up is the
+// faster one (66 heads of 16320 rows: 51.4 us with 7 splits, 46.6 with 8; 171
+// heads of 8128: 92 and 69; 257: 162 and 99; 384: 178 and 138; 450 heads of
+// 7300: 166 and 145).
 constexpr int kDecWaves = 512;
 constexpr int kDecMinTiles = 2;
 
 struct DecodeSplits {
   int S, kps;
 };
-static DecodeSplits decode_splits(int64_t heads, int C) {
+static DecodeSplits decode_splits(int64_t heads, int D, int C) {
   const int tiles = (C + kDecTile - 1) / kDecTile;
-  const int want = (int)std::max<int64_t>(1, std::min<int64_t>(kDecMaxSplits, kDecWaves / heads));
+  int64_t waves_per_head = kDecWaves / heads;
+  if (D == 64 && heads * waves_per_head < kDecWaves - kDecWaves / 16) ++waves_per_head;
+  const int want = (int)std::max<int64_t>(1, std::min<int64_t>(kDecMaxSplits, waves_per_head));
   const int per = std::max((tiles + want - 1) / want, std::min(tiles, kDecMinTiles));
   return DecodeSplits{(tiles + per - 1) / per, per * kDecTile};
 }
@@ -359,7 +369,7 @@ hipError_t launch_decode_attention(const DecodeParams& p, hipStream_t st) {
   a.Hkv = p.Hkv;
   a.D = p.D;
   a.C = p.C;
-  const DecodeSplits sp = decode_splits((int64_t)p.B * p.Hkv, p.C);
+  const DecodeSplits sp = decode_splits((int64_t)p.B * p.Hkv, p.D, p.C);
   a.S = sp.S;
   a.kps = sp.kps;
   a.scale_log2 = p.scale * 1.4426950408889634f;

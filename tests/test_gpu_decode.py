@@ -211,3 +211,31 @@ def test_tiles_and_splits(gpu, B, Hq, Hkv, D, C, n, aligned):
     # bf16 output: half an ulp (2^-9) of it, and the same of the weights' sum
     torch.testing.assert_close(out.float(), ref, rtol=2 ** -7, atol=2 ** -9)
     assert torch.equal(kb[:, :, n], kn[:, :, 0]) and torch.equal(vb[:, :, n], vn[:, :, 0])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("heads,n", [
+    (33, 700),   # 12 splits of three tiles, the last ones empty
+    (66, 288),   # 7 splits of five tiles (the last of four), the new row inside split 1
+    (171, 383), (171, 384),  # D = 64: 3 splits of 12 tiles, the new row at the end of split 0 and first in split 1
+    (257, 543), (257, 544),  # D = 64: 2 splits of 17 tiles, else one
+    (480, 1087), (481, 1056), (512, 0), (513, 1087),  # one split (D = 64, 479 heads and fewer: two)
+    (479, 544),
+])
+def test_heads_that_do_not_divide_the_waves(gpu, heads, n, D):
+    """Splits of 512 waves over any number of heads: rounded up at D = 64 where
+    a sixteenth of the waves or more would be missing."""
+    from dropkv_amd import ops
+    C, g = 1088, 2  # 34 tiles
+    gen = torch.Generator().manual_seed(heads + n)
+    kb, vb = (torch.randn(heads, 1, C, D, generator=gen).bfloat16().to(gpu) for _ in range(2))
+    kb[:, :, n:] = float("nan")
+    vb[:, :, n:] = float("nan")
+    q, kn, vn = (torch.randn(heads, h, 1, D, generator=gen).bfloat16().to(gpu) for h in (g, 1, 1))
+    k_rows, v_rows = (torch.cat([x[:, :, :n].clone(), y], dim=2) for x, y in ((kb, kn), (vb, vn)))
+    out = torch.empty(heads, 1, g, D, dtype=torch.bfloat16, device=gpu)
+    ops.decode_attention(q, kn, vn, kb, vb, torch.tensor([n], dtype=torch.int32, device=gpu), D ** -0.5, out,
+                         ops.decode_workspace(heads, g, 1, D, C, gpu))
+    # bf16 output: half an ulp (2^-9) of it, and the same of the weights' sum
+    torch.testing.assert_close(out.float(), _ref_attention(q, k_rows, v_rows, D ** -0.5), rtol=2 ** -7, atol=2 ** -9)
+    assert torch.equal(kb[:, :, n], kn[:, :, 0]) and torch.equal(vb[:, :, n], vn[:, :, 0])
