@@ -144,7 +144,10 @@ __global__ void __launch_bounds__(64) decode_partial_kernel(DecodeArgs a) {
   const int k1 = min(k0 + a.kps, n + 1);
   const bool own_n = k0 <= n && n < k1;  // this split holds the new row
 
-  float m = -INFINITY, lsum = 0.f;  // head li, log2 units; lsum is this lane's share
+  // Head li, log2 units; lsum is this lane's share.  The maximum starts finite, so
+  // that logits of -inf get no weight (-inf - -inf would be NaN) where a tile or
+  // the whole split has no other.
+  float m = -__FLT_MAX__, lsum = 0.f;
   f32x4 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -195,8 +198,8 @@ __global__ void __launch_bounds__(64) decode_partial_kernel(DecodeArgs a) {
         tmax = __builtin_elementwise_maximum(tmax, x);
       }
     tmax = max_xor32(max_xor16(tmax)) * a.scale_log2;
-    const float mnew = fmaxf(m, tmax);  // finite: key j0 is valid
-    const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mnew);
+    const float mnew = fmaxf(m, tmax);
+    const float alpha = __builtin_amdgcn_exp2f(m - mnew);
     // P^T operand: element e is key 4 lg + e (e < 4) or 16 + 4 lg + e - 4; the
     // transposing V reads below give V^T in that key order.
     float psum = 0.f;
@@ -278,8 +281,8 @@ __global__ void __launch_bounds__(64) decode_merge_kernel(DecodeArgs a) {
     ob[i] = __builtin_bit_cast(
           f32x4, __builtin_amdgcn_raw_buffer_load_b128(ors, ((uint32_t)(SPL * i + sub) * g * D + d0) * 4u, 0, 0));
   const float mx = wave_max_dpp(ml);
-  // Lanes past S, and splits with no rows, weigh 0.
-  const float f = ml == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml - mx);
+  // Lanes past S (-inf), and splits with no rows or none above -inf, weigh 0.
+  const float f = __builtin_amdgcn_exp2f(ml - mx);
   const float l = wave_sum_dpp(ll * f);
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -289,7 +292,7 @@ __global__ void __launch_bounds__(64) decode_merge_kernel(DecodeArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[e] = fmaf(fs, ob[i][e], acc[e]);
     }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = 1.f / l;  // (0 / 0 = NaN where every logit is -inf, as softmax gives)
   T* out = static_cast<T*>(a.out) + (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {

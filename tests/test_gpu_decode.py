@@ -239,3 +239,32 @@ def test_heads_that_do_not_divide_the_waves(gpu, heads, n, D):
     # bf16 output: half an ulp (2^-9) of it, and the same of the weights' sum
     torch.testing.assert_close(out.float(), _ref_attention(q, k_rows, v_rows, D ** -0.5), rtol=2 ** -7, atol=2 ** -9)
     assert torch.equal(kb[:, :, n], kn[:, :, 0]) and torch.equal(vb[:, :, n], vn[:, :, 0])
+
+
+@pytest.mark.parametrize("C,n,lo,hi", [
+    (4160, 4159, 0, 32),       # the first tile of a split
+    (4160, 4159, 96, 192),     # a whole split (96 rows)
+    (4160, 4159, 4128, 4159),  # the last split but its new row
+    (64, 40, 0, 40),           # everything but the new row
+    (64, 40, 0, 41),           # the new row too: NaN, as softmax gives
+    (200, 130, 5, 100),
+])
+@pytest.mark.parametrize("D", [64, 128])
+def test_logits_of_minus_infinity(gpu, C, n, lo, hi, D):
+    """Keys lo .. hi - 1 have logits of -inf and no weight, whole tiles and
+    splits of them included."""
+    from dropkv_amd import ops
+    g = torch.Generator().manual_seed(C + lo)
+    kb, vb = (torch.randn(1, 2, C, D, generator=g).bfloat16().to(gpu) for _ in range(2))
+    q, kn, vn = (torch.randn(1, h, 1, D, generator=g).bfloat16().to(gpu) for h in (8, 2, 2))
+    q[..., 0] = 1.0
+    kb[:, :, lo:hi, 0] = float("-inf")
+    if hi > n:
+        kn[..., 0] = float("-inf")
+    k_rows, v_rows = (torch.cat([x[:, :, :n].clone(), y], dim=2) for x, y in ((kb, kn), (vb, vn)))
+    out = torch.empty(1, 1, 8, D, dtype=torch.bfloat16, device=gpu)
+    ops.decode_attention(q, kn, vn, kb, vb, torch.tensor([n], dtype=torch.int32, device=gpu), D ** -0.5, out,
+                         ops.decode_workspace(1, 8, 2, D, C, gpu))
+    ref = _ref_attention(q, k_rows, v_rows, D ** -0.5)
+    assert torch.isfinite(ref).all() == (hi <= n)
+    torch.testing.assert_close(out.float(), ref, rtol=2 ** -7, atol=2 ** -9, equal_nan=True)
