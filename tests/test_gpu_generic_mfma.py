@@ -37,7 +37,7 @@ def _check(got, ref, rtol):
 
 @pytest.mark.parametrize("dtype,Hq,Hkv,D,Lk,W", [
     (torch.float32, 2, 2, 64, 256, 16),     # 16 rows: one row block; one step
-    (torch.float32, 2, 2, 64, 257, 17),     # 17 rows: two row blocks; a second split of one key
+    (torch.float32, 2, 2, 64, 257, 17),     # 17 rows: two row blocks; a second step of one key
     (torch.float32, 8, 2, 32, 255, 8),      # 32 rows
     (torch.float32, 7, 1, 128, 1000, 5),    # 35 rows: two chunks, the second of three rows
     (torch.float32, 4, 2, 36, 777, 3),      # 36 columns: a partial chunk, one group of y
@@ -89,3 +89,78 @@ def test_dominant_key_and_common_mean(gpu, dtype, D):
     q, k, v = _inputs(dtype, 1, 4, 2, D, W, Lk, seed=4, v_mean=100.0)
     ref = R.dropkv_scores_fp64(q, k, v, W)
     _check(ops.scores(q.to(gpu), k.to(gpu), v.to(gpu), W, p_round=False), ref, 1e-4)
+
+
+def test_many_splits_fp32(gpu):
+    """More than 32 key splits: the merge's second batch of partials."""
+    from dropkv_amd import ops
+    q, k, v = _inputs(torch.float32, 1, 2, 1, 64, 8, 17500, seed=11)
+    ref = R.dropkv_scores_fp64(q, k, v, 8)
+    for p_round in (False, True):  # (rounding to fp32 is the identity)
+        _check(ops.scores(q.to(gpu), k.to(gpu), v.to(gpu), 8, p_round=p_round), ref, 1e-4)
+
+
+def test_many_splits_rounded_p(gpu):
+    """70 key splits: each workgroup combines the statistics of more splits than
+    it reads up front.  Against the float64 score with p rounded: off by more
+    than 1e-4 only where a p rounds the other way (as test_rounded_p)."""
+    from dropkv_amd import ops
+    q, k, v = _inputs(torch.bfloat16, 1, 4, 1, 96, 8, 20000, seed=12)
+    got = ops.scores(q.to(gpu), k.to(gpu), v.to(gpu), 8, p_round=False, splits=78)
+    _check(got, R.dropkv_scores_fp64(q, k, v, 8), 1e-4)
+    ref = R.dropkv_scores_fp64(q, k, v, 8, p_round=torch.bfloat16)
+    got = ops.scores(q.to(gpu), k.to(gpu), v.to(gpu), 8, p_round=True, splits=78).double().cpu()
+    rel = (got - ref).abs() / ref.abs().clamp_min(1e-30)
+    assert rel.max() < 2e-2 and (rel > 1e-4).double().mean() < 2e-2
+
+
+@pytest.mark.parametrize("Lk", [4200, 4097])
+def test_several_tiles_a_wave_and_row_groups(gpu, Lk):
+    """More than 1024 workgroups of 64 keys: a wave takes several 16-key tiles,
+    and with 72 rows of 256 columns the rows are staged in groups, each key's
+    sum carried from one to the next."""
+    from dropkv_amd import ops
+    q, k, v = _inputs(torch.bfloat16, 1, 48, 16, 256, 24, Lk, seed=13)
+    args = q.to(gpu), k.to(gpu), v.to(gpu), 24
+    _check(ops.scores(*args, p_round=False), R.dropkv_scores_fp64(q, k, v, 24), 1e-4)
+    # p and y rounded (y's operands in 16 bits: groups of 64 rows), as the other
+    # tests of that path
+    got, ref = ops.scores(*args, y_round=True).cpu(), R.fallback_scores(q, k, v, 24)
+    torch.testing.assert_close(got, ref, rtol=2e-2, atol=1e-3)
+    rel = (got.double() - ref.double()).abs() / ref.double().abs().clamp_min(1e-30)
+    assert (rel > 1e-3).double().mean().item() < 1e-2
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 96), (torch.float16, 256)])
+@pytest.mark.parametrize("p_round", [False, True])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("key", [5, 700 - 8, 699])
+def test_value_that_is_not_finite(gpu, dtype, D, p_round, value, key):
+    """The last query row sees every key, so an infinite or NaN value in any row
+    of V leaves no finite score in its head, whichever of the other rows see it
+    (0 * inf is NaN in p @ V, as in torch); other heads are not touched."""
+    from dropkv_amd import ops
+    q, k, v = _inputs(dtype, 1, 6, 3, D, 8, 700, seed=14)
+    clean = ops.scores(q.to(gpu), k.to(gpu), v.to(gpu), 8, p_round=p_round).cpu()
+    v[0, 1, key, 3] = value
+    got = ops.scores(q.to(gpu), k.to(gpu), v.to(gpu), 8, p_round=p_round).cpu()
+    ref = R.dropkv_scores_reference(q, k, v, 8, match_pytorch_precision=p_round)
+    assert not torch.isfinite(ref[0, 1]).any() and not torch.isfinite(got[0, 1]).any()
+    assert torch.equal(got[:, ::2], clean[:, ::2]) and torch.isfinite(clean).all()
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 96)])
+@pytest.mark.parametrize("lo,hi", [(0, 1), (0, 256), (250, 700), (0, 1192), (1193, 1199)])
+def test_keys_of_minus_infinity(gpu, dtype, D, lo, hi):
+    """Keys whose logits are -inf have p = 0 and a score of 0; whole steps and
+    splits of them leave the other keys' scores alone."""
+    from dropkv_amd import ops
+    q, k, v = _inputs(dtype, 1, 4, 2, D, 8, 1200, seed=15)
+    q[..., 0] = 1.0
+    k[:, :, lo:hi, 0] = float("-inf")
+    ref = R.dropkv_scores_fp64(q, k, v, 8)
+    assert torch.isfinite(ref).all() and (ref[:, :, lo:hi] == 0).all()
+    got = ops.scores(q.to(gpu), k.to(gpu), v.to(gpu), 8, p_round=False)
+    # (few keys left: p up to 1 - delta, whose score is off by 2^-24 / delta)
+    _check(got, ref, 1e-3)
+    assert (got[:, :, lo:hi] == 0).all()
