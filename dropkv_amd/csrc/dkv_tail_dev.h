@@ -301,15 +301,21 @@ __device__ __forceinline__ void tail_emit(const SelFuse& fz, int row, int j0, in
   }
 }
 
-// The whole selection of one row whose scores one workgroup holds (sc, n =
-// Lk keys): the same rule as fused_tail with everything in LDS, so no
-// barriers between workgroups and nothing published.  The candidates (keys
-// inside the top-digit bin of the keep-th key) of a row this short are few:
-// up to kSoloRank of them are ranked against each other at once (a group of
-// threads per candidate), without a second digit.  Pass 2 of a 512-key layer-call
-// (2 rows, D = 64): 17.6 us in two workgroups per row with fused_tail, 11.9 in
-// one with this; 300 keys, one workgroup either way: 17.4 and 11.6.  L: tail_lds_words(NT, kps)
-// words of LDS (pass 2's operands are dead).
+// The whole selection of one row whose scores one workgroup holds (sc, Lk <=
+// kps <= kScLds keys): the same rule as fused_tail with everything in LDS, so
+// no barriers between workgroups and nothing published.  Rows of up to 512 keys
+// come here by the plan (plan_solo_rows), longer ones where a pass has one split:
+// more than 128 (batch, KV head) rows, or splits = 1.  Candidates are the keys
+// inside the top-digit bin of the keep-th key: up to kSoloRank of them, as in
+// short rows, are ranked against each other at once (a group of threads per
+// candidate), without a second digit; more go through the digits of fused_tail.
+// Pass 2 of a 512-key layer-call (2 rows, D = 64): 17.6 us in two workgroups per
+// row with fused_tail, 11.9 in one with this; 300 keys, one workgroup either way:
+// 17.4 and 11.6.  Layer-calls of 132 rows (D = 128, a tenth kept), fused_tail and
+// this: 800 keys 60.5 and 55.1 us, 2048 keys 99.1 and 92.7, 4096 keys 172.9 and
+// 162.4, half of 4096 kept 239.9 and 204.9; one split asked for, 16 rows of 4096
+// keys: 135.2 and 127.3.  L: tail_lds_words(NT, kps) words of LDS (pass 2's
+// operands are dead).
 constexpr uint32_t kSoloRank = 128;
 
 template <int NT>
