@@ -81,16 +81,22 @@ def test_decode_attention_strided_inputs(gpu):
 
 @pytest.mark.parametrize("D,Hq,Hkv", [(64, 14, 2), (128, 16, 1)])
 @pytest.mark.parametrize("C,n", [
-    (4160, 4159),   # 64 splits of 65 rows (two steps each, the second of one row); last row of the buffer
+    (4160, 4159),   # 44 splits of three tiles (96 rows), the last of one; last row of the buffer
+    (4160, 4128),   # the new row alone in the last split
+    (4160, 4127),   # the new row ends the last full split; the last one empty
     (4160, 4100),
-    (4160, 64),     # the new row alone in split 0's second step
-    (4160, 65),     # the new row first in split 1; splits 2.. empty
+    (4160, 97),
+    (4160, 96),     # the new row first in split 1; splits 2.. empty
+    (4160, 95),     # the new row ends split 0
+    (4160, 65),
+    (4160, 64),     # the new row first in split 0's third tile
     (4160, 0),      # only the new row
-    (200, 130),     # 4 splits of 50 rows: one partial step each
+    (200, 130),     # 4 splits of two tiles, the last one empty
+    (200, 192),     # the new row first in the last split, whose second tile lies past the buffer
 ])
 def test_decode_attention_split_edges_nan_rows(gpu, D, Hq, Hkv, C, n):
-    """Split rows are fixed by the capacity, so splits can run two steps,
-    end in a partial step, or hold no row at all. Every buffer row from the
+    """Split rows are fixed by the capacity, so splits can run several tiles,
+    end in a partial tile, or hold no row at all. Every buffer row from the
     new row's position on holds NaN: the rows past it are masked out of the
     logits and out of P.V (0 * NaN is NaN), and the buffer keeps them as
     they were; row n ends up holding the new row."""
@@ -190,7 +196,8 @@ def test_decoder_graph_replays_equal_eager_steps(gpu, tiny):
     (1, 4, 2, 128, 64, 31, False),     # the new row ends the first tile; scalar loads of q and the new row
     (1, 2, 1, 128, 4096, 4095, True),  # 64 splits of two tiles, buffer full
     (40, 16, 16, 64, 96, 70, True),    # 640 heads: one split each, the third tile partial
-    (3, 14, 2, 64, 2000, 1984, False),  # 32 splits of two tiles, the last ones empty
+    (3, 14, 2, 64, 2000, 1984, False),  # 32 splits of two tiles, the new row first in the last one
+    (3, 14, 2, 64, 2000, 1920, False),  # the new row first in a split that an empty one follows
 ])
 def test_tiles_and_splits(gpu, B, Hq, Hkv, D, C, n, aligned):
     """Edges of the 32-key tiles and of the splits (at least two tiles each),
