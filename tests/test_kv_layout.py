@@ -63,9 +63,20 @@ def test_route_misaligned_and_far_rows():
     d = flat[1:1 + B * H * L * 64].view(B, H, L, 64)
     u, _ = ops._evict_kv(d)
     assert u.data_ptr() % 16 == 0 and torch.equal(u, d)
-    # rows further apart than 32-bit offsets reach (no memory behind the view)
-    far = torch.empty(1, 1, 1, 64, dtype=torch.bfloat16, device="meta").as_strided((1, 1, 4096, 64), (8, 8, 1 << 19, 1))
-    assert far.stride(2) > (1 << 31) // 2 // (4096 + 1024)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_route_far_rows(dtype):
+    """Rows in place up to the distance that 32-bit offsets reach (2 GiB over the
+    head's rows and 1024 more), copied from one 16-byte unit beyond (views with
+    no memory behind them)."""
+    es, rows = dtype.itemsize, 4096
+    limit = (1 << 31) // es // (rows + 1024) // (16 // es) * (16 // es)
+    for sl, in_place in ((limit, True), (limit + 16 // es, False), (1 << 20, False)):
+        far = torch.empty(1, 1, 1, 64, dtype=dtype, device="meta").as_strided((1, 2, rows, 64), (128, 64, sl, 1))
+        u, strides = ops._evict_kv(far)
+        assert strides == ((128, 64, sl) if in_place else (2 * rows * 64, rows * 64, 64))
+        assert u.stride() == (far.stride() if in_place else (2 * rows * 64, rows * 64, 64, 1))
 
 
 @pytest.mark.parametrize("over,msg", [
