@@ -145,7 +145,9 @@ int dropkv_compact2(const void* k0, const void* v0, int64_t s0_b, int64_t s0_h, 
  * counters: they must be zero when a workspace is first used (fill a new
  * workspace with zeros), and every call leaves them zero.  The rest of the
  * workspace needs no initialisation.  Calls that share a workspace must be
- * serialised (one stream), as for every workspace here.
+ * serialised (one stream), as for every workspace here.  Its size does not
+ * always grow with Lk (longer rows can have fewer splits): a workspace for
+ * several shapes takes the largest of their sizes.
  * ------------------------------------------------------------------------ */
 #define DROPKV_SYNC_BYTES 4096
 size_t dropkv_evict_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Lk,
@@ -210,6 +212,18 @@ int dropkv_evict_noalloc(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss
  * buffers must not overlap the inputs.  With kv_ld = Lk and out_ld = keep it
  * is dropkv_evict.
  * ------------------------------------------------------------------------ */
+int dropkv_append(const void* k, const void* v, int64_t s_b, int64_t s_h, int64_t s_l, int64_t elem_bytes,
+                  int64_t B, int64_t H, int64_t L, int64_t D, void* k_dst, void* v_dst, int64_t dst_ld,
+                  int64_t row0, void* stream);
+
+int dropkv_evict_ld(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd,
+                    const void* k, const void* v, int64_t kv_ld, int dtype,
+                    int64_t B, int64_t Hq, int64_t Hkv, int64_t Lq, int64_t Lk, int64_t D,
+                    int64_t W, float eps, int p_round, int y_round, int64_t splits,
+                    int64_t kernel_size, int64_t protect_window, int64_t keep,
+                    float* scores, int64_t* keep_idx, void* k_out, void* v_out, int64_t out_ld,
+                    void* workspace, size_t workspace_bytes, void* stream);
+
 /* dropkv_evict_strided: dropkv_evict_ld on K/V of any layout with the D axis
  * contiguous: row l of (batch b, KV head h) starts at element b*k_sb + h*k_sh +
  * l*k_sl of k (v likewise), so that the [B, L, H, D] projections of a decoder
@@ -225,18 +239,6 @@ int dropkv_evict_strided(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss
                          int64_t kernel_size, int64_t protect_window, int64_t keep,
                          float* scores, int64_t* keep_idx, void* k_out, void* v_out, int64_t out_ld,
                          void* workspace, size_t workspace_bytes, void* stream);
-
-int dropkv_append(const void* k, const void* v, int64_t s_b, int64_t s_h, int64_t s_l, int64_t elem_bytes,
-                  int64_t B, int64_t H, int64_t L, int64_t D, void* k_dst, void* v_dst, int64_t dst_ld,
-                  int64_t row0, void* stream);
-
-int dropkv_evict_ld(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_sd,
-                    const void* k, const void* v, int64_t kv_ld, int dtype,
-                    int64_t B, int64_t Hq, int64_t Hkv, int64_t Lq, int64_t Lk, int64_t D,
-                    int64_t W, float eps, int p_round, int y_round, int64_t splits,
-                    int64_t kernel_size, int64_t protect_window, int64_t keep,
-                    float* scores, int64_t* keep_idx, void* k_out, void* v_out, int64_t out_ld,
-                    void* workspace, size_t workspace_bytes, void* stream);
 
 /* Where the layer-calls' selection runs (no counterpart in the reference,
  * whose pooling, top-k and gather are separate torch ops).  mode 1 (the
