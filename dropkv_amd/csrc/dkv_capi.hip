@@ -253,7 +253,7 @@ static int evict_impl(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, i
   dkv::ScorePlan p = dkv::make_score_plan(B, Hq, Hkv, Lk, D, W, splits);
   if (splits <= 0) dkv::plan_solo_rows(&p, Lk);
   const size_t s_bytes = ((size_t)B * Hkv * Lk * 4 + 255) & ~size_t(255);
-  const size_t need = p.total + s_bytes + dkv::select_workspace_bytes(B * Hkv, Lk);
+  const size_t need = dkv::evict_bytes(p, Lk);
   if (!workspace || workspace_bytes < need)
     return fail(DROPKV_E_WORKSPACE, "workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
   char* ws = static_cast<char*>(workspace);
@@ -429,6 +429,7 @@ int dropkv_append(const void* k, const void* v, int64_t s_b, int64_t s_h, int64_
 }
 
 static_assert(DROPKV_SYNC_BYTES == dkv::kSyncBytes, "the header's sync area is the plan's");
+static_assert(DROPKV_NOALLOC_SCRATCH_BYTES == dkv::kNoallocBytes, "the header's static scratch is the plan's");
 
 int dropkv_set_tail_select(int mode, int64_t spin_polls, int64_t spin_polls_b) {
   if (mode != 0 && mode != 1) return fail(DROPKV_E_ARG, "mode must be 0 or 1");

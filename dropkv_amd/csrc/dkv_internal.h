@@ -134,6 +134,12 @@ size_t decode_workspace_bytes(int B, int Hq, int Hkv, int D, int C);
 hipError_t launch_decode_attention(const DecodeParams& p, hipStream_t st);
 
 size_t select_workspace_bytes(int64_t rows, int64_t Lk);
+// Workspace of a layer-call: the plan's, the scores and the selection's.
+inline size_t evict_bytes(const ScorePlan& p, int64_t Lk) {
+  return p.total + (((size_t)p.heads * Lk * 4 + 255) & ~size_t(255)) + select_workspace_bytes(p.heads, Lk);
+}
+// The static scratch of dropkv_evict_noalloc.
+constexpr size_t kNoallocBytes = size_t(32) << 20;
 // Words at the start of the selection workspace that must be zero on entry
 // (cleared by launch_select itself unless the caller already did it).
 int64_t select_zero_words(int64_t rows);

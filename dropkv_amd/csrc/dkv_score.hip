@@ -1156,8 +1156,10 @@ static inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b)
 #define DKV_P2_WIDE_GROUP 3    // tiles per LDS stage of the wide pass 2 (1 to 3)
 #endif
 
-ScorePlan make_score_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Lk, int64_t D, int64_t W,
-                          int64_t splits) {
+// The plan of make_score_plan; fill: pass 1 of two row-chunks on every CU, where
+// the call is one that gains by it.
+static ScorePlan score_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Lk, int64_t D, int64_t W, int64_t splits,
+                            bool fill) {
   ScorePlan p;
   p.heads = (int)(B * Hkv);
   p.g = (int)(Hq / Hkv);
@@ -1185,17 +1187,16 @@ ScorePlan make_score_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Lk, int64_
   // the merge still combines at most kMergeFew partials in one round (D=128,
   // W=16, B=2 Hkv=8 at Lk 32768: 177 -> 154 us per layer-call; B=1 at 16384:
   // 61.7 -> 57.3; B=5 at 8192: 125 -> 111; B=12 at 3001: the same).
-  // Up to 2^20 keys in all: the extra partials must not push a call that fits
-  // the 32 MiB of the no-allocation entry point over them.  At the tuned head
-  // dimensions they are 2 MB at most, and the scratch 29 MB with them.  The
-  // partials grow with D: with the rule at every D, calls of D = 256 to 1024
-  // that the entry point takes were refused (B=1 Hq=32 Hkv=8 D=1024 W=16 at Lk
-  // 4096: 26.4 -> 38.5 MiB), and above D = 256 no kernel reads them.
+  // Up to D = 256, above which no kernel reads the partials, and up to 2^20 keys
+  // in all: the extra partials (2 MB at most at the tuned head dimensions, whose
+  // scratch is then at most 29 MB) must not push a call that fits the 32 MiB of
+  // the no-allocation entry point over them; make_score_plan has the larger
+  // head dimensions.
   constexpr int kMergeFew = 64;
   constexpr int64_t kFillKeys = int64_t(1) << 20;
   const int target1 = (p1_bw && !p.p1_wide) ? DKV_TARGET_P1_BW : target;
   int s1 = splits > 0 ? (int)splits : ceil_div(target1, p1_groups);
-  if (splits <= 0 && p1_bw && !p.p1_wide && p.n_mc > 1 && mfma_head_dim(D) && p.heads * Lk <= kFillKeys)
+  if (fill && splits <= 0 && p1_bw && !p.p1_wide && p.n_mc > 1 && D <= 256 && p.heads * Lk <= kFillKeys)
     s1 = max(s1, min(kMergeFew, (int)(target / p1_groups)));
   s1 = max(1, min(min(s1, max_by_work), kMaxSplits));
   p.kps1 = ceil_div(ceil_div(Lk, s1), kTile) * kTile;
@@ -1225,6 +1226,20 @@ ScorePlan make_score_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Lk, int64_
   p.off_yf = take((size_t)p.heads * p.mpad * D * sizeof(float));
   p.total = off;
   return p;
+}
+
+// The partials grow with D: at D = 256 the extra ones can push a layer-call that
+// the static scratch of the no-allocation entry point holds over it (B=20 Hq=32
+// Hkv=2 W=4 at Lk 24390: 29.9 -> 32.5 MiB).  Such a call keeps the fewer splits.
+// Outside the tuned head dimensions filling the CUs takes a fifth off a call (B=1
+// Hq=32 Hkv=8 W=16, scores alone, us: D=256 at Lk 8192 123.5 -> 99.6, at 32768
+// 368 -> 290; D=96 at 32768 190 -> 150; D=192 at 16384 176 -> 136).
+ScorePlan make_score_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Lk, int64_t D, int64_t W,
+                          int64_t splits) {
+  const ScorePlan p = score_plan(B, Hq, Hkv, Lk, D, W, splits, true);
+  if (mfma_head_dim(D) || evict_bytes(p, Lk) <= kNoallocBytes) return p;
+  const ScorePlan few = score_plan(B, Hq, Hkv, Lk, D, W, splits, false);
+  return evict_bytes(few, Lk) <= kNoallocBytes ? few : p;
 }
 
 bool kv_rows_fit(int64_t row_stride, int64_t elem_bytes, int64_t Lk, int64_t D) {
